@@ -83,9 +83,9 @@ __device__ __forceinline__ int cascade_prefix_groups(int tp, int ts, int G, int 
 // 32-row tiles, no workgroup combine) and the suffix body's.
 constexpr int kCascadeMergeLdsSeqs = 1024;
 
-template <int D, int RS> union MfmaLdsPair {
-    MfmaLds<D, 2, 0> a;
-    MfmaLds<D, RS> b;
+template <int KV, int D, int RS> union MfmaLdsPair {
+    MfmaLds<KV, D, 2, 0> a;
+    MfmaLds<KV, D, RS> b;
 };
 
 // Partition launch over both batches.  pp / ps are the prefix and suffix
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, 2) void paged_decode_casca
     const int *__restrict__ stables) {
     constexpr int NW = kMfmaWavesPerGroup;
     extern __shared__ int pre[];  // prefix batch (pp.num_seqs + 1), then suffix batch
-    __shared__ MfmaLdsPair<D, RS> sm;
+    __shared__ MfmaLdsPair<KV, D, RS> sm;
     int *pre_p = pre, *pre_s = pre + pp.num_seqs + 1;
     batch_prefix<16, NW>(pp, pre_p);
     batch_prefix<16, NW>(ps, pre_s);
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, 2) void paged_decode_casca
     const int *__restrict__ pblocks, int num_groups, int *__restrict__ p_row) {
     constexpr int NW = kMfmaWavesPerGroup, NT = 64 * NW;
     extern __shared__ int lds[];
-    __shared__ MfmaLdsPair<D, RS> sm;
+    __shared__ MfmaLdsPair<KV, D, RS> sm;
     __shared__ int s_part[NW];
     __shared__ int s_win[NW][2 * kMfmaHeads];  // prefix pieces' members (mfma_load_q)
     const int B = ps.num_seqs, V = pp.num_seqs, NG = num_groups;

@@ -111,7 +111,7 @@ static hipError_t launch_for_head_size(const DecodeParams &p, int head_tile, boo
                     paged_decode_partition_mfma_kernel<KV, D, 1>, mgrid, 64 * kMfmaWavesPerGroup,
                     lds, st, ev_start, ev_stop, p, p.seq_lens, p.block_tables);
                 if (e != hipSuccess) return e;
-                return launch_merge<KV, D, kMfmaHeads, MfmaGeometry<D>::kTile>(p, st);
+                return launch_merge<KV, D, kMfmaHeads, MfmaGeometry<KV, D>::kTile>(p, st);
             }
             if constexpr (has_mfma_wide<KV, D>()) {
                 if (head_tile == 2 * kMfmaHeads) {
@@ -120,7 +120,7 @@ static hipError_t launch_for_head_size(const DecodeParams &p, int head_tile, boo
                         64 * kMfmaWavesPerGroup, lds, st, ev_start, ev_stop, p, p.seq_lens,
                         p.block_tables);
                     if (e != hipSuccess) return e;
-                    return launch_merge<KV, D, 2 * kMfmaHeads, MfmaGeometry<D>::kTile>(p, st);
+                    return launch_merge<KV, D, 2 * kMfmaHeads, MfmaGeometry<KV, D>::kTile>(p, st);
                 }
             }
         }

@@ -3,30 +3,41 @@
 // query heads of one kv head (R = 1, or 2 for groups of 17-32 heads at
 // head_size <= 128): every K/V tile it loads is used by all 16R heads.
 // Below, one row block; with R = 2 the QK^T MFMAs run once per block on the
-// same K registers, and each V^T operand read from LDS feeds both blocks' PV
-// MFMAs.
+// same K registers, and each V^T operand feeds both blocks' PV MFMAs.
 //
 // Per 16-token tile (one page when block_size = 16), with g = lane/16 and
 // j = lane%16 (v_mfma_f32_16x16x{32,16} operand layouts, checked on gfx950):
 //   QK^T  S[token][head] = sum_d K[token][d] Q[head][d]
-//         D/32 x v_mfma_f32_16x16x32: A = K rows (lane: token j, dims
+//         D/32 x v_mfma_f32_16x16x32: A = K rows (lane: row j, dims
 //         32c+8g..+7, a 16-byte load straight from the page), B = Q of the 16
-//         heads (lane: head j, same dims).  C: lane holds S[4g+r][j].
+//         heads (lane: head j, same dims).  C: lane holds rows 4g+r of head j.
+//         Row 4g+r is token tile_token(g, r) = 4r+g.
 //   softmax per head j: the 16 scores of head j sit in lanes j, j+16, j+32,
 //         j+48 (4 each): in-lane max, two xor shuffles, exp2, running sum.
 //   PV    O^T[dim][head] += sum_t V[t][dim] P[head][t]
-//         D/16 x v_mfma_f32_16x16x16 (twice: P = P_hi + P_lo in the 16-bit
-//         type, so the product keeps ~22 bits of P): B = P, which is exactly
-//         the C layout of the QK^T step (lane: head j, tokens 4g..4g+3);
-//         A = V^T (lane: dim 16n+j, tokens 4g..4g+3), read from the V tile
-//         staged in LDS.  C: lane holds O^T[16n+4g+r][j].
-// The V tile goes global -> registers -> LDS (row stride 2*D+8 bytes so the
-// four token groups of a V^T read fall in different LDS banks).  Loads are
-// buffer loads: a token past the end of the range, or in a page with a
-// negative id, gets an out-of-range offset and reads as zero without touching
-// memory; its score is masked to -inf.  The next tile's K/V loads are issued
-// before the current tile is computed.
+//         v_mfma_f32_16x16x16 per dim block (twice: P = P_hi + P_lo in the
+//         16-bit type, so the product keeps ~22 bits of P): B = P, which is
+//         exactly the C layout of the QK^T step (lane: head j, rows
+//         4g..4g+3); A = V^T (lane: one dim per block, the same four tokens).
+//         Which dim a lane holds in which block is free, so lane (g, j) loads
+//         chunk j of each of its own four token rows (16 bytes at
+//         head_size 128; the row in 16 equal chunks below that, and in groups
+//         of 16 above), and the dims of a chunk become row j of as many
+//         blocks.  V goes from the load registers to the MFMA with two
+//         v_perm_b32 per block (one half of each of four rows), and C (lane:
+//         O^T rows 4g+r of head j) holds a chunk's consecutive dims over the
+//         blocks of its group: whole output chunks.
+//         A trip of the tile through LDS instead (row-major write, 32
+//         two-byte reads a lane to gather V^T) was 40 LDS instructions and a
+//         write-to-read wait in every tile's chain; fp16, head_size 128,
+//         16 x 1024 tokens, 32 / 8 heads: 21.3 -> 20.7 us a step.
+// Loads are buffer loads: a token past the end of the range, or in a page
+// with a negative id, gets an out-of-range offset and reads as zero without
+// touching memory; its score is masked to -inf.  The next tile's K/V loads
+// are issued before the current tile is computed.
 #pragma once
+
+#include <type_traits>
 
 #include "paged_decode_kernels.h"
 #include "wg_trace.h"
@@ -37,19 +48,40 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 
 constexpr uint32_t kOobOffset = 0x80000000u;
 
-template <int D> struct MfmaGeometry {
-    static constexpr int kTile = 16;             // tokens per tile
-    static constexpr int kChunks = D / 8;        // 16-byte chunks per 16-bit row
-    static constexpr int kQkSteps = D / 32;      // QK^T MFMAs = K loads per lane
-    static constexpr int kVLoads = D / 32;       // V 16-byte loads per lane (16 rows)
-    static constexpr int kDimBlocks = D / 16;    // PV MFMAs per P half
-    static constexpr int kLdsRow = 2 * D + 8;    // bytes per staged V row
-    static constexpr int kLdsTile = 16 * kLdsRow;
+template <int KV, int D> struct MfmaGeometry {
+    static constexpr int kTile = 16;  // tokens per tile
+    static constexpr int kElemBytes = KvTraits<KV>::kBytes;
+    static constexpr int kRowBytes = kElemBytes * D;
+    static constexpr int kQkSteps = (kRowBytes + 63) / 64;  // 16-byte K loads per lane
+    // V rows: groups of 16 chunks, a lane holding one chunk of each group (of
+    // its four token rows); full groups have kDims dims (16 bytes) per chunk,
+    // the last one as many as the row still has.
+    static constexpr int kDims = 16 / kElemBytes;
+    static constexpr int kVGroups = (D + 16 * kDims - 1) / (16 * kDims);
+    static constexpr int group_dims(int b) {
+        return (D - 16 * kDims * b) / 16 < kDims ? (D - 16 * kDims * b) / 16 : kDims;
+    }
+    static constexpr int group_words(int b) { return group_dims(b) * kElemBytes / 4; }
+    static constexpr int kDimBlocks = kDims * (kVGroups - 1) + group_dims(kVGroups - 1);
+    // Rows of fewer than 16 chunks of 16 bytes: the tile is loaded in whole
+    // 16-byte lanes and dealt to the lane chunks through LDS (4- to 12-byte
+    // loads, one per token row, are slower: head_size 32, bf16, 64 sequences
+    // of 256-4096 tokens, 32 / 8 heads 39.4 us a step).
+    static constexpr bool kVStaged = kRowBytes < 256;
+    static constexpr int kVLoads = kVStaged ? kRowBytes / 64 : 4 * kVGroups;
     static_assert(D % 32 == 0, "MFMA path needs head_size % 32 == 0");
 };
+
+// First of the group_dims(b) dims of chunk i of V group b: element e of the
+// chunk is row i of dim block kDims * b + e.
+template <int KV, int D> __device__ __forceinline__ int mfma_dim(int b, int i) {
+    using G = MfmaGeometry<KV, D>;
+    return 16 * G::kDims * b + G::group_dims(b) * i;
+}
 
 template <int KV> __device__ __forceinline__ f32x4 mfma_qk(u32x4 a, u32x4 b, f32x4 c) {
     if constexpr (KV == KV_F16)
@@ -79,82 +111,184 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const char *base) {
 // 4 KB runs, 16-byte lane loads) from ~5.9 to ~6.6 TB/s.
 constexpr int kStreamPolicy = 2;
 
-__device__ __forceinline__ u32x4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, kStreamPolicy);
+// A chunk of W words (1 to 4; the rest of the vector is unspecified).
+template <int W, int POLICY>
+__device__ __forceinline__ u32x4 buf_load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    u32x4 x;
+    if constexpr (W == 4) {
+        x = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, POLICY);
+    } else if constexpr (W == 3) {
+        const u32x3 y = __builtin_amdgcn_raw_buffer_load_b96(r, (int)off, 0, POLICY);
+        x = __builtin_shufflevector(y, y, 0, 1, 2, -1);
+    } else if constexpr (W == 2) {
+        const u32x2 y = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, POLICY);
+        x = __builtin_shufflevector(y, y, 0, 1, -1, -1);
+    } else {
+        x.x = __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, POLICY);
+    }
+    return x;
 }
 
-__device__ __forceinline__ u32x4 buf_load16_cached(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+// fn(std::integral_constant<int, b>) for every V group b (their widths differ).
+template <int KV, int D, typename Fn> __device__ __forceinline__ void for_groups(Fn &&fn) {
+    constexpr int N = MfmaGeometry<KV, D>::kVGroups;
+    static_assert(N >= 1 && N <= 4, "V groups of a row");
+    fn(std::integral_constant<int, 0>{});
+    if constexpr (N > 1) fn(std::integral_constant<int, 1>{});
+    if constexpr (N > 2) fn(std::integral_constant<int, 2>{});
+    if constexpr (N > 3) fn(std::integral_constant<int, 3>{});
 }
 
-template <int D> struct MfmaTileRegs {
-    u32x4 k[MfmaGeometry<D>::kQkSteps];
-    u32x4 v[MfmaGeometry<D>::kVLoads];
+template <int KV, int D> struct MfmaTileRegs {
+    u32x4 k[MfmaGeometry<KV, D>::kQkSteps];     // score row j, 16 bytes at 64c + 16g of the K row
+    u32x4 v[MfmaGeometry<KV, D>::kVLoads];      // 4b + r: score row 4g + r, chunk j of V group b;
+                                                // staged: bytes 1024c + 16 * lane of the V tile
 };
+
+// Token, within its tile, of score row 4g + r.  Lane group g holds V rows
+// tile_token(g, 0..3), one per load, so a load covers the four neighbouring
+// rows 4r..4r+3.  (With rows 4g + r, 4 apart in a load, the pieces of a row
+// that is not whole 128-byte lines were fetched twice: head_size 96, 24
+// sequences of 100-2000 tokens, 32 / 32 heads 60.1 us against 57.)
+__device__ __forceinline__ int tile_token(int g, int r) { return 4 * r + g; }
+
+template <int KV, int D, int POLICY>
+__device__ __forceinline__ void mfma_issue_loads(__amdgpu_buffer_rsrc_t rk,
+                                                 __amdgpu_buffer_rsrc_t rv, int n, int lane,
+                                                 MfmaTileRegs<KV, D> &r) {
+    using G = MfmaGeometry<KV, D>;
+    constexpr int RB = G::kRowBytes;
+    const int j = lane & 15, g = lane >> 4;
+    const int kt = tile_token(j >> 2, j & 3);
+    const bool krow_ok = kt < n;
+#pragma unroll
+    for (int c = 0; c < G::kQkSteps; c++)
+        r.k[c] = buf_load<4, POLICY>(rk, krow_ok ? (uint32_t)(kt * RB + 64 * c + 16 * g) : kOobOffset);
+    if constexpr (G::kVStaged) {
+#pragma unroll
+        for (int c = 0; c < G::kVLoads; c++) {
+            const int at = 1024 * c + 16 * lane;
+            r.v[c] = buf_load<4, POLICY>(rv, at / RB < n ? (uint32_t)at : kOobOffset);
+        }
+    } else {
+        for_groups<KV, D>([&](auto b) {
+            constexpr int B = decltype(b)::value;
+            constexpr int W = G::group_words(B);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                r.v[4 * B + i] = buf_load<W, POLICY>(
+                    rv, tile_token(g, i) < n
+                            ? (uint32_t)(tile_token(g, i) * RB + 256 * B + 4 * W * j)
+                            : kOobOffset);
+        });
+    }
+}
 
 // Issue the K and V loads of the tile starting at token t0 (block id blk):
 // rows past t_end or in a negative page read as zero.
-template <int D>
+template <int KV, int D>
 __device__ __forceinline__ void mfma_load_tile(const DecodeParams &p, const char *kb,
                                                const char *vb, int t0, int t_end, int blk,
-                                               int lane, bool cached, MfmaTileRegs<D> &r) {
-    using G = MfmaGeometry<D>;
+                                               int lane, bool cached, MfmaTileRegs<KV, D> &r) {
+    constexpr int EB = MfmaGeometry<KV, D>::kElemBytes;
     const int bmask = p.block_size - 1;
-    const bool page_ok = blk >= 0;
     const long long page = (long long)blk * p.kv_block_stride + (long long)(t0 & bmask) * D;
-    const __amdgpu_buffer_rsrc_t rk = tile_rsrc(kb + page * 2);
-    const __amdgpu_buffer_rsrc_t rv = tile_rsrc(vb + page * 2);
-    const int j = lane & 15, g = lane >> 4;
-    const bool krow_ok = page_ok && (t0 + j < t_end);
-    uint32_t koff[G::kQkSteps], voff[G::kVLoads];
-#pragma unroll
-    for (int c = 0; c < G::kQkSteps; c++)
-        koff[c] = krow_ok ? (uint32_t)(j * 2 * D + 64 * c + 16 * g) : kOobOffset;
-#pragma unroll
-    for (int c = 0; c < G::kVLoads; c++) {
-        const int q = 64 * c + lane;
-        const int row = q / G::kChunks;
-        const int chunk = q - row * G::kChunks;
-        const bool ok = page_ok && (t0 + row < t_end);
-        voff[c] = ok ? (uint32_t)(row * 2 * D + 16 * chunk) : kOobOffset;
-    }
-    if (cached) {
-#pragma unroll
-        for (int c = 0; c < G::kQkSteps; c++) r.k[c] = buf_load16_cached(rk, koff[c]);
-#pragma unroll
-        for (int c = 0; c < G::kVLoads; c++) r.v[c] = buf_load16_cached(rv, voff[c]);
-    } else {
-#pragma unroll
-        for (int c = 0; c < G::kQkSteps; c++) r.k[c] = buf_load16(rk, koff[c]);
-#pragma unroll
-        for (int c = 0; c < G::kVLoads; c++) r.v[c] = buf_load16(rv, voff[c]);
-    }
+    const __amdgpu_buffer_rsrc_t rk = tile_rsrc(kb + page * EB);
+    const __amdgpu_buffer_rsrc_t rv = tile_rsrc(vb + page * EB);
+    const int n = blk >= 0 ? t_end - t0 : 0;  // tokens of the tile
+    if (cached)
+        mfma_issue_loads<KV, D, 0>(rk, rv, n, lane, r);
+    else
+        mfma_issue_loads<KV, D, kStreamPolicy>(rk, rv, n, lane, r);
 }
 
 // Running state of one wavefront over one segment: lane (g, j) owns head j.
-template <int D> struct MfmaState {
-    f32x4 o[MfmaGeometry<D>::kDimBlocks];  // O^T[16n + 4g + r][j]
+template <int KV, int D> struct MfmaState {
+    f32x4 o[MfmaGeometry<KV, D>::kDimBlocks];  // block kDims*b + e, row 4g + r of
+                                               // head j: dim mfma_dim(b, 4g + r) + e
     float m;                               // running max of head j (log2 units)
     float l;                               // this lane's part of the running sum
 };
 
-template <int KV, int D, int R>
-__device__ __forceinline__ void mfma_tile(const DecodeParams &p, const u32x4 (*q)[MfmaGeometry<D>::kQkSteps],
-                                          int t0, int t_end, bool page_ok, int lane, char *lds,
-                                          const MfmaTileRegs<D> &r, MfmaState<D> (&st)[R]) {
-    using G = MfmaGeometry<D>;
-    const int j = lane & 15, g = lane >> 4;
+// A piece's query rows (MFMA B layout): in registers, or, where R = 2 states
+// leave no room for them beside two tiles of K/V (head_size 128: 10 VGPRs
+// spilled, and 64 / 2 heads over 64 sequences of 512-8192 tokens took 76.7 us
+// against 67.0), parked by each lane in LDS and read back every tile.
+template <int KV, int D, int R> constexpr bool mfma_q_in_lds() {
+    return R == 2 && MfmaGeometry<KV, D>::kRowBytes > 128;
+}
+template <int KV, int D, int R, bool LDS = mfma_q_in_lds<KV, D, R>()> struct MfmaQLds {};
+template <int KV, int D, int R> struct MfmaQLds<KV, D, R, true> {
+    u32x4 q[R][MfmaGeometry<KV, D>::kQkSteps][64];
+};
 
-    // V tile -> LDS (row-major, padded rows), two 8-byte writes per chunk.
-#pragma unroll
-    for (int c = 0; c < G::kVLoads; c++) {
-        const int qi = 64 * c + lane;
-        const int row = qi / G::kChunks;
-        const int chunk = qi - row * G::kChunks;
-        u32x2 *dst = (u32x2 *)(lds + row * G::kLdsRow + 16 * chunk);
-        dst[0] = u32x2{r.v[c][0], r.v[c][1]};
-        dst[1] = u32x2{r.v[c][2], r.v[c][3]};
+// The V tile of a wavefront where it is staged (MfmaGeometry::kVStaged), row-major.
+template <int KV, int D, bool STAGED = MfmaGeometry<KV, D>::kVStaged> struct MfmaVLds {
+    __device__ __forceinline__ void put(const MfmaTileRegs<KV, D> &, int) {}
+    // chunk j of V group B of the lane's score row 4g + i
+    template <int B>
+    __device__ __forceinline__ u32x4 chunk(const MfmaTileRegs<KV, D> &r, int, int i) const {
+        return r.v[4 * B + i];
     }
+};
+template <int KV, int D> struct MfmaVLds<KV, D, true> {
+    u32x4 t[64 * MfmaGeometry<KV, D>::kVLoads];
+    __device__ __forceinline__ void put(const MfmaTileRegs<KV, D> &r, int lane) {
+#pragma unroll
+        for (int c = 0; c < MfmaGeometry<KV, D>::kVLoads; c++) t[64 * c + lane] = r.v[c];
+    }
+    template <int B>
+    __device__ __forceinline__ u32x4 chunk(const MfmaTileRegs<KV, D> &, int lane, int i) const {
+        using G = MfmaGeometry<KV, D>;
+        constexpr int W = G::group_words(B);
+        const uint32_t *src = (const uint32_t *)t +
+                              tile_token(lane >> 4, i) * (G::kRowBytes / 4) + W * (lane & 15);
+        u32x4 x;
+        if constexpr (W == 2) {
+            const u32x2 y = *(const u32x2 *)src;
+            x = __builtin_shufflevector(y, y, 0, 1, -1, -1);
+        } else {
+#pragma unroll
+            for (int w = 0; w < W; w++) x[w] = src[w];
+        }
+        return x;
+    }
+};
+
+template <int KV, int D, int R, bool LDS = mfma_q_in_lds<KV, D, R>()> struct MfmaQuery {
+    u32x4 q[R][MfmaGeometry<KV, D>::kQkSteps];
+    __device__ __forceinline__ void put(MfmaQLds<KV, D, R> &, int,
+                                        const u32x4 (&x)[R][MfmaGeometry<KV, D>::kQkSteps]) {
+#pragma unroll
+        for (int b = 0; b < R; b++)
+#pragma unroll
+            for (int c = 0; c < MfmaGeometry<KV, D>::kQkSteps; c++) q[b][c] = x[b][c];
+    }
+    __device__ __forceinline__ u32x4 get(const MfmaQLds<KV, D, R> &, int, int b, int c) const {
+        return q[b][c];
+    }
+};
+template <int KV, int D, int R> struct MfmaQuery<KV, D, R, true> {
+    __device__ __forceinline__ void put(MfmaQLds<KV, D, R> &s, int lane,
+                                        const u32x4 (&x)[R][MfmaGeometry<KV, D>::kQkSteps]) {
+#pragma unroll
+        for (int b = 0; b < R; b++)
+#pragma unroll
+            for (int c = 0; c < MfmaGeometry<KV, D>::kQkSteps; c++) s.q[b][c][lane] = x[b][c];
+    }
+    __device__ __forceinline__ u32x4 get(const MfmaQLds<KV, D, R> &s, int lane, int b, int c) const {
+        return s.q[b][c][lane];
+    }
+};
+
+template <int KV, int D, int R>
+__device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery<KV, D, R> &q,
+                                          int t0, int t_end, bool page_ok, int lane,
+                                          const MfmaQLds<KV, D, R> &qs, MfmaVLds<KV, D> &vs,
+                                          const MfmaTileRegs<KV, D> &r, MfmaState<KV, D> (&st)[R]) {
+    using G = MfmaGeometry<KV, D>;
+    const int g = lane >> 4;
+    vs.put(r, lane);
 
     // S = K Q^T for 16 tokens x 16 heads, per row block.
     f32x4 s[R];
@@ -163,13 +297,13 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const u32x4 (*q
 #pragma unroll
     for (int c = 0; c < G::kQkSteps; c++)
 #pragma unroll
-        for (int b = 0; b < R; b++) s[b] = mfma_qk<KV>(r.k[c], q[b][c], s[b]);
+        for (int b = 0; b < R; b++) s[b] = mfma_qk<KV>(r.k[c], q.get(qs, lane, b, c), s[b]);
 
     bool ok[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) ok[i] = page_ok && (t0 + 4 * g + i < t_end);
+    for (int i = 0; i < 4; i++) ok[i] = page_ok && (t0 + tile_token(g, i) < t_end);
 
-    // Online softmax of head j over tokens 4g..4g+3 of this lane; P in the
+    // Online softmax of head j over the four tokens of this lane; P in the
     // 16-bit type as hi + lo parts (B operand of the PV MFMA).
     u32x2 p_hi[R], p_lo[R];
 #pragma unroll
@@ -207,21 +341,87 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const u32x4 (*q
         }
     }
 
-    // O^T += V^T P for every 16-dim block.
-    const char *vrow = lds + (4 * g) * G::kLdsRow + 2 * j;
+    // O^T += V^T P for every dim block: the block's dim of the lane's four
+    // token rows, a 16-bit half of one word of each row's chunk.
+    for_groups<KV, D>([&](auto vb) {
+        constexpr int B = decltype(vb)::value;
+        u32x4 v[4];
 #pragma unroll
-    for (int n = 0; n < G::kDimBlocks; n++) {
-        const char *src = vrow + 32 * n;
-        const uint32_t v0 = *(const uint16_t *)(src);
-        const uint32_t v1 = *(const uint16_t *)(src + G::kLdsRow);
-        const uint32_t v2 = *(const uint16_t *)(src + 2 * G::kLdsRow);
-        const uint32_t v3 = *(const uint16_t *)(src + 3 * G::kLdsRow);
-        const u32x2 a = {v0 | (v1 << 16), v2 | (v3 << 16)};
+        for (int i = 0; i < 4; i++) v[i] = vs.template chunk<B>(r, lane, i);
 #pragma unroll
-        for (int b = 0; b < R; b++) {
-            st[b].o[n] = mfma_pv<KV>(a, p_hi[b], st[b].o[n]);
-            st[b].o[n] = mfma_pv<KV>(a, p_lo[b], st[b].o[n]);
+        for (int e = 0; e < G::group_dims(B); e++) {
+            const int n = G::kDims * B + e, w = e / 2;
+            const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+            const u32x2 a = {__builtin_amdgcn_perm(lane_word(v[1], w), lane_word(v[0], w), sel),
+                             __builtin_amdgcn_perm(lane_word(v[3], w), lane_word(v[2], w), sel)};
+#pragma unroll
+            for (int b = 0; b < R; b++) {
+                st[b].o[n] = mfma_pv<KV>(a, p_hi[b], st[b].o[n]);
+                st[b].o[n] = mfma_pv<KV>(a, p_lo[b], st[b].o[n]);
+            }
         }
+    });
+}
+
+// The lane's dims of row i = 4g + r of V group B (consecutive ones from
+// mfma_dim(B, i)), gathered from the blocks of a state.
+template <int KV, int D, int B>
+__device__ __forceinline__ void state_dims(const MfmaState<KV, D> &st, int r,
+                                           float (&f)[MfmaGeometry<KV, D>::group_dims(B)]) {
+    using G = MfmaGeometry<KV, D>;
+#pragma unroll
+    for (int e = 0; e < G::group_dims(B); e++) f[e] = st.o[G::kDims * B + e][r];
+}
+
+// N consecutive floats of a row whose first one is at a multiple of N (N = 4
+// or 8: 16-byte aligned; else of the largest power of two in N).
+template <int N> constexpr int float_step() { return N % 4 == 0 ? 4 : N % 2 == 0 ? 2 : 1; }
+
+template <int N> __device__ __forceinline__ void store_floats(float *dst, const float (&f)[N]) {
+    constexpr int S = float_step<N>();
+#pragma unroll
+    for (int e = 0; e < N; e += S) {
+        if constexpr (S == 4) *(f32x4 *)(dst + e) = f32x4{f[e], f[e + 1], f[e + 2], f[e + 3]};
+        else if constexpr (S == 2) *(f32x2 *)(dst + e) = f32x2{f[e], f[e + 1]};
+        else dst[e] = f[e];
+    }
+}
+
+template <int N> __device__ __forceinline__ void load_floats(const float *src, float (&f)[N]) {
+    constexpr int S = float_step<N>();
+#pragma unroll
+    for (int e = 0; e < N; e += S) {
+        if constexpr (S == 4) {
+            const f32x4 x = *(const f32x4 *)(src + e);
+#pragma unroll
+            for (int k = 0; k < 4; k++) f[e + k] = x[k];
+        } else if constexpr (S == 2) {
+            const f32x2 x = *(const f32x2 *)(src + e);
+            f[e] = x.x;
+            f[e + 1] = x.y;
+        } else {
+            f[e] = src[e];
+        }
+    }
+}
+
+// N consecutive values of the element type at element d of a row (d a
+// multiple of N), rounded to nearest even.
+template <int KV, int N>
+__device__ __forceinline__ void store_elems(char *row, int d, const float (&f)[N]) {
+    if constexpr (KV == KV_F32) {
+        store_floats((float *)row + d, f);
+    } else {
+        static_assert(N % 2 == 0, "16-bit elements go in pairs");
+        uint32_t w[N / 2];
+#pragma unroll
+        for (int e = 0; e < N / 2; e++) w[e] = pack16<KV>(f[2 * e], f[2 * e + 1]);
+        uint32_t *dst = (uint32_t *)(row + (size_t)d * 2);
+        if constexpr (N == 8) *(u32x4 *)dst = u32x4{w[0], w[1], w[2], w[3]};
+        else if constexpr (N == 4) *(u32x2 *)dst = u32x2{w[0], w[1]};
+        else
+#pragma unroll
+            for (int e = 0; e < N / 2; e++) dst[e] = w[e];
     }
 }
 
@@ -344,9 +544,9 @@ __device__ __forceinline__ bool next_piece(const DecodeParams &p, const int *__r
 // members of its rows with one ballot per 64 caller sequences, and the piece
 // that starts its sequence's kv head 0 stores each member's first row
 // (p_row).
-template <int D, int R, int SRC = kSrcBatch>
+template <int KV, int D, int R, int SRC = kSrcBatch>
 __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPiece &pc, int lane,
-                                            u32x4 (&q)[R][MfmaGeometry<D>::kQkSteps],
+                                            u32x4 (&q)[R][MfmaGeometry<KV, D>::kQkSteps],
                                             const CascadeLdsPlan *cp = nullptr) {
     const int j = lane & 15, g = lane >> 4;
     const int g0 = pc.ht * kMfmaHeads * R;
@@ -387,7 +587,7 @@ __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPie
                 if (first && gq == 0 && g == 0) cp->p_row[s] = vbase * cp->rows + r * G;
             }
 #pragma unroll
-            for (int c = 0; c < MfmaGeometry<D>::kQkSteps; c++)
+            for (int c = 0; c < MfmaGeometry<KV, D>::kQkSteps; c++)
                 q[b][c] = src ? load16(src + (size_t)(32 * c + 8 * g) * 2) : u32x4{0, 0, 0, 0};
         }
         return;
@@ -397,7 +597,7 @@ __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPie
 #pragma unroll
     for (int b = 0; b < R; b++)
 #pragma unroll
-        for (int c = 0; c < MfmaGeometry<D>::kQkSteps; c++)
+        for (int c = 0; c < MfmaGeometry<KV, D>::kQkSteps; c++)
             q[b][c] = (16 * b + j < nh)
                           ? load16(q0 + ((size_t)(16 * b + j) * D + 32 * c + 8 * g) * 2)
                           : u32x4{0, 0, 0, 0};
@@ -409,15 +609,16 @@ __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPie
 // tile, like one more partial.  Its loads are issued when the piece begins
 // (R = 1), so their latency hides behind the piece's tiles; with R = 2 the 32
 // extra registers would not fit, and they are loaded at the end.
-template <int D, int R> struct MfmaFold {
-    f32x4 o[R][MfmaGeometry<D>::kDimBlocks];
+template <int KV, int D, int R> struct MfmaFold {
+    f32x4 o[R][MfmaGeometry<KV, D>::kDimBlocks];
     float m[R];
     int base;  // the sequence's fold base, < 0: no fold
 };
 
-template <int D, int R>
+template <int KV, int D, int R>
 __device__ __forceinline__ void mfma_fold_load(const DecodeParams &p, const MfmaPiece &pc,
-                                               int lane, MfmaFold<D, R> &f) {
+                                               int lane, MfmaFold<KV, D, R> &f) {
+    using G = MfmaGeometry<KV, D>;
     const int j = lane & 15, g = lane >> 4;
     const int g0 = pc.ht * kMfmaHeads * R;
     const int nh = min(kMfmaHeads * R, p.group - g0);
@@ -426,15 +627,22 @@ __device__ __forceinline__ void mfma_fold_load(const DecodeParams &p, const Mfma
         // heads past the group read head g0 (valid) and are never written
         const size_t r = fold_state_row(p, f.base, pc.kvh, g0 + (16 * b + j < nh ? 16 * b + j : 0));
         f.m[b] = p.fold_lse[r];
+        for_groups<KV, D>([&](auto vb) {
+            constexpr int B = decltype(vb)::value, N = G::group_dims(B);
 #pragma unroll
-        for (int n = 0; n < MfmaGeometry<D>::kDimBlocks; n++)
-            f.o[b][n] = *(const f32x4 *)(p.fold_out + r * D + 16 * n + 4 * g);
+            for (int i = 0; i < 4; i++) {
+                float x[N];
+                load_floats(p.fold_out + r * D + mfma_dim<KV, D>(B, 4 * g + i), x);
+#pragma unroll
+                for (int e = 0; e < N; e++) f.o[b][G::kDims * B + e][i] = x[e];
+            }
+        });
     }
 }
 
-template <int D, int R>
-__device__ __forceinline__ void mfma_fold_apply(const MfmaFold<D, R> &f, int lane,
-                                                MfmaState<D> (&st)[R]) {
+template <int KV, int D, int R>
+__device__ __forceinline__ void mfma_fold_apply(const MfmaFold<KV, D, R> &f, int lane,
+                                                MfmaState<KV, D> (&st)[R]) {
     const int g = lane >> 4;
 #pragma unroll
     for (int b = 0; b < R; b++) {
@@ -443,7 +651,7 @@ __device__ __forceinline__ void mfma_fold_apply(const MfmaFold<D, R> &f, int lan
         const float a = fast_exp2(st[b].m - Ms), w = fast_exp2(f.m[b] - Ms);
         st[b].l = st[b].l * a + (g == 0 ? w : 0.0f);  // l is summed over the 4 lane groups
 #pragma unroll
-        for (int n = 0; n < MfmaGeometry<D>::kDimBlocks; n++)
+        for (int n = 0; n < MfmaGeometry<KV, D>::kDimBlocks; n++)
             st[b].o[n] = st[b].o[n] * a + f.o[b][n] * w;
         st[b].m = M;
     }
@@ -469,8 +677,8 @@ namespace xhip {
 // per-lane sums (lane group g of head j); they are reduced here.
 template <int KV, int D, int R, bool HS = false>
 __device__ __forceinline__ void mfma_write_rows(const DecodeParams &p, const MfmaPiece &pc,
-                                                int lane, const MfmaState<D> (&st)[R]) {
-    using G = MfmaGeometry<D>;
+                                                int lane, const MfmaState<KV, D> (&st)[R]) {
+    using G = MfmaGeometry<KV, D>;
     constexpr int GT = kMfmaHeads * R;
     const int j = lane & 15, gq = lane >> 4;
     const int g0 = pc.ht * GT;
@@ -484,38 +692,36 @@ __device__ __forceinline__ void mfma_write_rows(const DecodeParams &p, const Mfm
         const int hj = 16 * b + j;  // head of this lane in the tile
         if (hj >= nh) continue;
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        if constexpr (HS) {
-            char *dst = (char *)p.out_h + (qrow0 + (size_t)hj * D + 4 * gq) * 2;
+        const size_t row = qrow0 + (size_t)hj * D;  // element index
+        char *orow = HS          ? (char *)p.out_h + row * 2
+                     : p.out_f32 ? (char *)(p.out_f32 + row)
+                                 : o_row(p, pc.s, pc.kvh * p.group + g0 + hj, D, G::kElemBytes);
+        for_groups<KV, D>([&](auto vb) {
+            constexpr int B = decltype(vb)::value, N = G::group_dims(B);
 #pragma unroll
-            for (int n = 0; n < G::kDimBlocks; n++) {
-                const f32x4 o = st[b].o[n] * inv;
-                *(u32x2 *)(dst + 32 * n) =
-                    u32x2{pack16<KV_F16>(o[0], o[1]), pack16<KV_F16>(o[2], o[3])};
+            for (int i = 0; i < 4; i++) {
+                const int d = mfma_dim<KV, D>(B, 4 * gq + i);
+                float f[N];
+                state_dims<KV, D, B>(st[b], i, f);
+#pragma unroll
+                for (int e = 0; e < N; e++) f[e] *= inv;
+                if constexpr (HS) store_elems<KV_F16>(orow, d, f);
+                else if (p.out_f32) store_floats((float *)orow + d, f);
+                else store_elems<KV>(orow, d, f);
             }
-            if (gq == 0) p.out_lse[qrow0 / D + hj] = l > 0.0f ? st[b].m + log2f(l) : -INFINITY;
-        } else if (p.out_f32) {
-            float *dst = p.out_f32 + qrow0 + (size_t)hj * D + 4 * gq;
-#pragma unroll
-            for (int n = 0; n < G::kDimBlocks; n++) *(f32x4 *)(dst + 16 * n) = st[b].o[n] * inv;
-            if (gq == 0) p.out_lse[qrow0 / D + hj] = l > 0.0f ? st[b].m + log2f(l) : -INFINITY;
-        } else {
-            char *dst = o_row(p, pc.s, pc.kvh * p.group + g0 + hj, D, 2) + 4 * gq * 2;
-#pragma unroll
-            for (int n = 0; n < G::kDimBlocks; n++) {
-                const f32x4 o = st[b].o[n] * inv;
-                *(u32x2 *)(dst + 32 * n) = u32x2{pack16<KV>(o[0], o[1]), pack16<KV>(o[2], o[3])};
-            }
-        }
+        });
+        if ((HS || p.out_f32) && gq == 0)
+            p.out_lse[qrow0 / D + hj] = l > 0.0f ? st[b].m + log2f(l) : -INFINITY;
     }
 }
 
 // The partial of a cut segment's piece, in the piece's slot of the split-K
 // workspace: fp32 (m, l, unnormalized o), or HS: an fp16 state
 // (DecodeParams::ws_h) (m + log2 l, 1, o / l in fp16).
-template <int D, int R, bool HS = false>
+template <int KV, int D, int R, bool HS = false>
 __device__ __forceinline__ void mfma_write_partial(const DecodeParams &p, const MfmaPiece &pc,
-                                                   int lane, const MfmaState<D> (&st)[R]) {
-    using G = MfmaGeometry<D>;
+                                                   int lane, const MfmaState<KV, D> (&st)[R]) {
+    using G = MfmaGeometry<KV, D>;
     constexpr int GT = kMfmaHeads * R;
     const int j = lane & 15, gq = lane >> 4;
     const int nh = min(GT, p.group - pc.ht * GT);
@@ -526,28 +732,28 @@ __device__ __forceinline__ void mfma_write_partial(const DecodeParams &p, const 
         l += __shfl_xor(l, 32);
         const int hj = 16 * b + j;
         if (hj >= nh) continue;
-        if constexpr (HS) {
-            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-            char *dst = (char *)p.ws_h + (((size_t)pc.slot * GT + hj) * D + 4 * gq) * 2;
+        const float inv = !HS ? 1.0f : l > 0.0f ? 1.0f / l : 0.0f;
+        const size_t row = ((size_t)pc.slot * GT + hj) * D;
+        for_groups<KV, D>([&](auto vb) {
+            constexpr int B = decltype(vb)::value, N = G::group_dims(B);
 #pragma unroll
-            for (int n = 0; n < G::kDimBlocks; n++) {
-                const f32x4 o = st[b].o[n] * inv;
-                *(u32x2 *)(dst + 32 * n) =
-                    u32x2{pack16<KV_F16>(o[0], o[1]), pack16<KV_F16>(o[2], o[3])};
-            }
-            if (gq == 0) {
-                p.ws_ml[((size_t)pc.slot * GT + hj) * 2] =
-                    l > 0.0f ? st[b].m + log2f(l) : -INFINITY;
-                p.ws_ml[((size_t)pc.slot * GT + hj) * 2 + 1] = l > 0.0f ? 1.0f : 0.0f;
-            }
-            continue;
-        }
-        float *dst = p.ws_o + ((size_t)pc.slot * GT + hj) * D + 4 * gq;
+            for (int i = 0; i < 4; i++) {
+                const int d = mfma_dim<KV, D>(B, 4 * gq + i);
+                float f[N];
+                state_dims<KV, D, B>(st[b], i, f);
+                if constexpr (HS) {
 #pragma unroll
-        for (int n = 0; n < G::kDimBlocks; n++) *(f32x4 *)(dst + 16 * n) = st[b].o[n];
+                    for (int e = 0; e < N; e++) f[e] *= inv;
+                    store_elems<KV_F16>((char *)p.ws_h + row * 2, d, f);
+                } else {
+                    store_floats(p.ws_o + row + d, f);
+                }
+            }
+        });
         if (gq == 0) {
-            p.ws_ml[((size_t)pc.slot * GT + hj) * 2] = st[b].m;
-            p.ws_ml[((size_t)pc.slot * GT + hj) * 2 + 1] = l;
+            float *ml = p.ws_ml + ((size_t)pc.slot * GT + hj) * 2;
+            ml[0] = !HS ? st[b].m : l > 0.0f ? st[b].m + log2f(l) : -INFINITY;
+            ml[1] = !HS ? l : l > 0.0f ? 1.0f : 0.0f;
         }
     }
 }
@@ -555,73 +761,76 @@ __device__ __forceinline__ void mfma_write_partial(const DecodeParams &p, const 
 // LDS slot of one wavefront for the workgroup-level combine (mfma_wg_fixup):
 // a state in the lane layout of MfmaState (per-lane o, m and unreduced l),
 // so two states merge lane by lane.
-template <int D> struct MfmaFixSlot {
-    f32x4 o[MfmaGeometry<D>::kDimBlocks][64];
+template <int KV, int D> struct MfmaFixSlot {
+    f32x4 o[MfmaGeometry<KV, D>::kDimBlocks][64];
     float m[64], l[64];
     int ends;  // the state reaches the end of its segment
 };
 
-template <int D>
-__device__ __forceinline__ void fix_store(MfmaFixSlot<D> &slot, int lane, const MfmaState<D> &st) {
+template <int KV, int D>
+__device__ __forceinline__ void fix_store(MfmaFixSlot<KV, D> &slot, int lane, const MfmaState<KV, D> &st) {
 #pragma unroll
-    for (int n = 0; n < MfmaGeometry<D>::kDimBlocks; n++) slot.o[n][lane] = st.o[n];
+    for (int n = 0; n < MfmaGeometry<KV, D>::kDimBlocks; n++) slot.o[n][lane] = st.o[n];
     slot.m[lane] = st.m;
     slot.l[lane] = st.l;
 }
 
-template <int D>
-__device__ __forceinline__ void fix_load(const MfmaFixSlot<D> &slot, int lane, MfmaState<D> &st) {
+template <int KV, int D>
+__device__ __forceinline__ void fix_load(const MfmaFixSlot<KV, D> &slot, int lane, MfmaState<KV, D> &st) {
 #pragma unroll
-    for (int n = 0; n < MfmaGeometry<D>::kDimBlocks; n++) st.o[n] = slot.o[n][lane];
+    for (int n = 0; n < MfmaGeometry<KV, D>::kDimBlocks; n++) st.o[n] = slot.o[n][lane];
     st.m = slot.m[lane];
     st.l = slot.l[lane];
 }
 
 // st <- st (+) the state in slot (online log-sum-exp, per lane).
-template <int D>
-__device__ __forceinline__ void fix_absorb(const MfmaFixSlot<D> &slot, int lane, MfmaState<D> &st) {
+template <int KV, int D>
+__device__ __forceinline__ void fix_absorb(const MfmaFixSlot<KV, D> &slot, int lane, MfmaState<KV, D> &st) {
     const float mo = slot.m[lane];
     const float M = fmaxf(st.m, mo);
     const float Ms = (M == -INFINITY) ? 0.0f : M;
     const float a = fast_exp2(st.m - Ms), b = fast_exp2(mo - Ms);
     st.l = st.l * a + slot.l[lane] * b;
 #pragma unroll
-    for (int n = 0; n < MfmaGeometry<D>::kDimBlocks; n++) st.o[n] = st.o[n] * a + slot.o[n][lane] * b;
+    for (int n = 0; n < MfmaGeometry<KV, D>::kDimBlocks; n++) st.o[n] = st.o[n] * a + slot.o[n][lane] * b;
     st.m = M;
 }
 
 // The workgroup's relay slot of the mode-2 combine: one state of R row
 // blocks in the lane layout, and per wavefront whether it relayed its state
 // there (and whether that state reaches the end of its segment).
-template <int D, int R> struct MfmaRelaySlot {
-    f32x4 o[R][MfmaGeometry<D>::kDimBlocks][64];
+template <int KV, int D, int R> struct MfmaRelaySlot {
+    f32x4 o[R][MfmaGeometry<KV, D>::kDimBlocks][64];
     float m[R][64], l[R][64];
     int relayed[kMfmaWavesPerGroup];
     int ends[kMfmaWavesPerGroup];
 };
 
-// LDS of one workgroup of the partition kernel: the V tile staging of each
-// wavefront, and the slots of the workgroup-level combine (by mode).
-template <int FIX, int D, int R> struct MfmaSweepLds {
+// LDS of one workgroup of the partition kernel: the query rows of
+// each wavefront's piece (R = 2), its V tile (short rows), and the slots of the workgroup-level combine (by
+// mode).
+template <int FIX, int KV, int D, int R> struct MfmaSweepLds {
     int unused;
 };
-template <int D, int R> struct MfmaSweepLds<1, D, R> {
-    MfmaFixSlot<D> fix[kMfmaWavesPerGroup];
+template <int KV, int D, int R> struct MfmaSweepLds<1, KV, D, R> {
+    MfmaFixSlot<KV, D> fix[kMfmaWavesPerGroup];
 };
-template <int D, int R> struct MfmaSweepLds<2, D, R> {
-    MfmaRelaySlot<D, R> relay;
+template <int KV, int D, int R> struct MfmaSweepLds<2, KV, D, R> {
+    MfmaRelaySlot<KV, D, R> relay;
 };
-template <int D, int R, int FIX = mfma_wg_fixup(kMfmaHeads * R, D)> struct MfmaLds {
-    __attribute__((aligned(16))) char vtile[kMfmaWavesPerGroup][MfmaGeometry<D>::kLdsTile];
-    MfmaSweepLds<FIX, D, R> sw;
+template <int KV, int D, int R, int FIX = mfma_wg_fixup(kMfmaHeads * R, D)> struct MfmaLds {
+    MfmaQLds<KV, D, R> qs[kMfmaWavesPerGroup];
+    MfmaVLds<KV, D> vs[kMfmaWavesPerGroup];
+    MfmaSweepLds<FIX, KV, D, R> sw;
 };
 
 // st <- st (+) the partial in workspace slot `slot` (its l is the reduced
 // sum: lane group 0 takes it; fp32, or HS: an fp16 state).  Rows past the group
 // were never written; they are left alone.
-template <int D, int R, bool HS = false>
+template <int KV, int D, int R, bool HS = false>
 __device__ __forceinline__ void absorb_partial(const DecodeParams &p, int slot, int ht, int lane,
-                                               MfmaState<D> (&st)[R]) {
+                                               MfmaState<KV, D> (&st)[R]) {
+    using G = MfmaGeometry<KV, D>;
     constexpr int GT = kMfmaHeads * R;
     const int j = lane & 15, gq = lane >> 4;
     const int nh = min(GT, p.group - ht * GT);
@@ -629,16 +838,37 @@ __device__ __forceinline__ void absorb_partial(const DecodeParams &p, int slot, 
     for (int b = 0; b < R; b++) {
         const int hj = 16 * b + j;
         if (hj >= nh) continue;
-        const size_t at = ((size_t)slot * GT + hj) * D + 4 * gq;
+        const size_t row = ((size_t)slot * GT + hj) * D;
         const float mo = p.ws_ml[((size_t)slot * GT + hj) * 2];
         const float lo = gq == 0 ? p.ws_ml[((size_t)slot * GT + hj) * 2 + 1] : 0.0f;
         const float M = fmaxf(st[b].m, mo);
         const float Ms = (M == -INFINITY) ? 0.0f : M;
         const float a = fast_exp2(st[b].m - Ms), w = fast_exp2(mo - Ms);
         st[b].l = st[b].l * a + lo * w;
+        for_groups<KV, D>([&](auto vb) {
+            constexpr int B = decltype(vb)::value, N = G::group_dims(B);
 #pragma unroll
-        for (int n = 0; n < MfmaGeometry<D>::kDimBlocks; n++)
-            st[b].o[n] = st[b].o[n] * a + partial_f32x4<HS>(p, at + 16 * n) * w;
+            for (int i = 0; i < 4; i++) {
+                const size_t at = row + mfma_dim<KV, D>(B, 4 * gq + i);
+                float x[N];
+                if constexpr (HS) {
+#pragma unroll
+                    for (int e = 0; e < N; e += 2) {
+                        const f32x2 h =
+                            unpack16<KV_F16>(*(const uint32_t *)((const char *)p.ws_h + (at + e) * 2));
+                        x[e] = h.x;
+                        x[e + 1] = h.y;
+                    }
+                } else {
+                    load_floats(p.ws_o + at, x);
+                }
+#pragma unroll
+                for (int e = 0; e < N; e++) {
+                    f32x4 &o = st[b].o[G::kDims * B + e];
+                    o[i] = o[i] * a + x[e] * w;
+                }
+            }
+        });
         st[b].m = M;
     }
 }
@@ -691,14 +921,13 @@ template <int KV, int D, int R, bool PAIR = false, int SRC = kSrcBatch, bool HS 
 __device__ __forceinline__ void mfma_partition_body(
     const DecodeParams &p, const int *__restrict__ lens, const int *__restrict__ tables,
     const int *pre, int wg, int waves,
-    MfmaLds<D, R, PAIR ? 0 : mfma_wg_fixup(kMfmaHeads * R, D)> &sm,
+    MfmaLds<KV, D, R, PAIR ? 0 : mfma_wg_fixup(kMfmaHeads * R, D)> &sm,
     const CascadeLdsPlan *cp = nullptr) {
-    using G = MfmaGeometry<D>;
+    using G = MfmaGeometry<KV, D>;
     constexpr int FIX = PAIR ? 0 : mfma_wg_fixup(kMfmaHeads * R, D);
     constexpr int NW = kMfmaWavesPerGroup;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    char *lds = sm.vtile[wave];
     if constexpr (FIX == 2) {
         // ordered before any read by the sweep's first barrier
         if (lane == 0) sm.sw.relay.relayed[wave] = 0;
@@ -711,7 +940,7 @@ __device__ __forceinline__ void mfma_partition_body(
     const int tpw = tiles_per_wave(total, PAIR ? waves >> 1 : waves, p.min_tiles_per_wave);
     const long long g_lo = (long long)wr * tpw;
 
-    MfmaState<D> st[R];   // the state of the piece being computed; after the loop, the last one's
+    MfmaState<KV, D> st[R];   // the state of the piece being computed; after the loop, the last one's
     MfmaPiece pc;         // the piece being computed; after the loop, the last one
     bool have_last = false;  // FIX: the last piece is cut (its state is kept for the sweep)
     MfmaPiece pc_first;      // FIX == 1, first wavefront: its cut first piece, saved in its slot
@@ -740,25 +969,27 @@ __device__ __forceinline__ void mfma_partition_body(
     // A range inside one segment's start-up units holds no tile (only when
     // tpw <= seg_cost); the segment's tiles belong to the next wavefront.
     if (g_lo < total && next_piece<16, SRC>(p, lens, pre, cur, pc, cp)) {
-        u32x4 q[R][G::kQkSteps];
+        u32x4 ql[R][G::kQkSteps];
+        MfmaQuery<KV, D, R> q;
         int ids;
         if constexpr (SRC == kSrcPrefix) {
             // (the block ids' round trip overlaps the members' lookup)
             ids = mfma_load_ids<SRC>(p, tables, pc, 0, lane, cp);
-            mfma_load_q<D, R, SRC>(p, pc, lane, q, cp);
+            mfma_load_q<KV, D, R, SRC>(p, pc, lane, ql, cp);
         } else {
-            mfma_load_q<D, R, SRC>(p, pc, lane, q, cp);
+            mfma_load_q<KV, D, R, SRC>(p, pc, lane, ql, cp);
             ids = mfma_load_ids<SRC>(p, tables, pc, 0, lane, cp);
         }
+        q.put(sm.qs[wave], lane, ql);
         // fold base of the current piece (requested a piece ahead from here on)
         int fold_base = (p.fold_row && pc.t_begin == 0) ? p.fold_row[pc.s] : -1;
-        MfmaTileRegs<D> ra, rb;
+        MfmaTileRegs<KV, D> ra, rb;
         int blk_a = __builtin_amdgcn_readlane(ids, 0);
         XHIP_WAVE_STAMP(p, wave, 0);
         {
             const char *kb = (const char *)p.k + (size_t)pc.kvh * (size_t)p.kv_head_stride * 2;
             const char *vb = (const char *)p.v + (size_t)pc.kvh * (size_t)p.kv_head_stride * 2;
-            mfma_load_tile<D>(p, kb, vb, pc.t_begin, pc.t_end, blk_a, lane, pc.s < p.cached_seqs,
+            mfma_load_tile<KV, D>(p, kb, vb, pc.t_begin, pc.t_end, blk_a, lane, pc.s < p.cached_seqs,
                               ra);
         }
 
@@ -787,9 +1018,9 @@ __device__ __forceinline__ void mfma_partition_body(
                 st[b].m = -INFINITY;
                 st[b].l = 0.0f;
             }
-            MfmaFold<D, R> fold;
+            MfmaFold<KV, D, R> fold;
             fold.base = fold_base;
-            if (R == 1 && fold.base >= 0) mfma_fold_load<D, R>(p, pc, lane, fold);
+            if (R == 1 && fold.base >= 0) mfma_fold_load<KV, D, R>(p, pc, lane, fold);
             const int ntiles = (pc.t_end - pc.t_begin + 15) >> 4;
 #if XHIP_TRACING
             n_tiles += ntiles;
@@ -807,18 +1038,18 @@ __device__ __forceinline__ void mfma_partition_body(
                     blk_b = nl != 0 ? __builtin_amdgcn_readlane(ids, nl) : bt[(t0 + 16) >> p.bs_shift];
                 else
                     blk_b = has_next ? __builtin_amdgcn_readlane(ids_n, 0) : -1;
-                mfma_load_tile<D>(p, in_piece ? kb : kb_n, in_piece ? vb : vb_n,
+                mfma_load_tile<KV, D>(p, in_piece ? kb : kb_n, in_piece ? vb : vb_n,
                                   in_piece ? t0 + 16 : pn.t_begin,
                                   in_piece ? pc.t_end : (has_next ? pn.t_end : 0), blk_b, lane,
                                   in_piece ? cached : cached_n, rb);
-                mfma_tile<KV, D, R>(p, q, t0, pc.t_end, blk_a >= 0, lane, lds, ra, st);
+                mfma_tile<KV, D, R>(p, q, t0, pc.t_end, blk_a >= 0, lane, sm.qs[wave], sm.vs[wave], ra, st);
                 ra = rb;
                 blk_a = blk_b;
             }
 
             if (fold.base >= 0) {
-                if (R != 1) mfma_fold_load<D, R>(p, pc, lane, fold);
-                mfma_fold_apply<D, R>(fold, lane, st);
+                if (R != 1) mfma_fold_load<KV, D, R>(p, pc, lane, fold);
+                mfma_fold_apply<KV, D, R>(fold, lane, st);
             }
             if (pc.whole) {
                 mfma_write_rows<KV, D, R, HS>(p, pc, lane, st);
@@ -830,7 +1061,7 @@ __device__ __forceinline__ void mfma_partition_body(
                     // (whose left neighbour is in another workgroup) is
                     // written as a partial after the range, so that its
                     // stores do not sit in front of the next piece's loads.
-                    fix_store<D>(sm.sw.fix[wave], lane, st[0]);
+                    fix_store<KV, D>(sm.sw.fix[wave], lane, st[0]);
                     if (lane == 0) sm.sw.fix[wave].ends = 1;
                     if (wave == 0) {
                         pc_first = pc;
@@ -841,17 +1072,18 @@ __device__ __forceinline__ void mfma_partition_body(
                 }
             } else if constexpr (FIX == 2) {
                 if (has_next)
-                    mfma_write_partial<D, R, HS>(p, pc, lane, st);
+                    mfma_write_partial<KV, D, R, HS>(p, pc, lane, st);
                 else
                     have_last = true;
             } else {
-                mfma_write_partial<D, R, HS>(p, pc, lane, st);
+                mfma_write_partial<KV, D, R, HS>(p, pc, lane, st);
             }
             if (!has_next) break;
             pc = pn;
             ids = ids_n;
             fold_base = fold_base_n;
-            mfma_load_q<D, R, SRC>(p, pc, lane, q, cp);
+            mfma_load_q<KV, D, R, SRC>(p, pc, lane, ql, cp);
+            q.put(sm.qs[wave], lane, ql);
         }
         XHIP_WAVE_STAMP(p, wave, 1);
     }
@@ -885,7 +1117,7 @@ __device__ __forceinline__ void mfma_partition_body(
                         // the neighbour's first piece, followed by more
                         // pieces, was written as a partial in its slot 0;
                         // it ends the segment in that range
-                        absorb_partial<D, R, HS>(p, (w + 1) * 2, pc.ht, lane, st);
+                        absorb_partial<KV, D, R, HS>(p, (w + 1) * 2, pc.ht, lane, st);
                         ends = true;
                     }
                 }
@@ -904,7 +1136,7 @@ __device__ __forceinline__ void mfma_partition_body(
                 } else if (!cut_start && ends) {
                     mfma_write_rows<KV, D, R, HS>(p, pc, lane, st);
                 } else {
-                    mfma_write_partial<D, R, HS>(p, pc, lane, st);
+                    mfma_write_partial<KV, D, R, HS>(p, pc, lane, st);
                 }
             }
             __syncthreads();
@@ -921,25 +1153,25 @@ __device__ __forceinline__ void mfma_partition_body(
         // finished rows when it lay in the workgroup, else one partial.
         const bool cut_start = have_last && pc.t_begin > 0;
         if (have_last && cut_start && wave > 0) {
-            fix_store<D>(sm.sw.fix[wave], lane, st[0]);
+            fix_store<KV, D>(sm.sw.fix[wave], lane, st[0]);
             if (lane == 0) sm.sw.fix[wave].ends = pc.t_end >= pc.L ? 1 : 0;
         }
         __syncthreads();
         if (first_saved) {
-            MfmaState<D> sf[R];
-            fix_load<D>(sm.sw.fix[0], lane, sf[0]);
-            mfma_write_partial<D, R, HS>(p, pc_first, lane, sf);
+            MfmaState<KV, D> sf[R];
+            fix_load<KV, D>(sm.sw.fix[0], lane, sf[0]);
+            mfma_write_partial<KV, D, R, HS>(p, pc_first, lane, sf);
         }
         if (have_last && !(cut_start && wave > 0)) {
             bool ends = pc.t_end >= pc.L;
             for (int j = wave + 1; !ends && j < NW; j++) {
-                fix_absorb<D>(sm.sw.fix[j], lane, st[0]);
+                fix_absorb<KV, D>(sm.sw.fix[j], lane, st[0]);
                 ends = sm.sw.fix[j].ends != 0;
             }
             if (!cut_start && ends)
                 mfma_write_rows<KV, D, R, HS>(p, pc, lane, st);
             else
-                mfma_write_partial<D, R, HS>(p, pc, lane, st);
+                mfma_write_partial<KV, D, R, HS>(p, pc, lane, st);
         }
     }
 }
@@ -954,7 +1186,7 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, D <= 128 ? 2 : 1) void pag
     // kernel arguments their wavefront-uniform reads become scalar loads,
     // which do not wait behind the K/V loads in flight.
     extern __shared__ int pre[];  // num_seqs + 1 split-unit prefixes
-    __shared__ MfmaLds<D, R> sm;
+    __shared__ MfmaLds<KV, D, R> sm;
     XHIP_WG_BEGIN(p);
     batch_prefix<16, kMfmaWavesPerGroup>(p, pre);
     XHIP_WG_STAMP(p, 1);
