@@ -501,7 +501,7 @@ int run(void *out, const void *query, const void *key_cache, const void *value_c
         const size_t eb_total = (size_t)elem_bytes(kv_dtype);
         // workspace: fp32 partials o, their (m, l), the unit prefix; under a
         // split segment launch, one partial per workgroup
-        const size_t pre_bytes = seg_launch ? 0 : (size_t)(nseq + 1) * sizeof(int);
+        const size_t pre_bytes = seg_launch ? 0 : (size_t)(nseq + 2) * sizeof(int);
         long long slots = seg_launch ? (seg_split > 1 ? nseq * segs * seg_split : 0)
                                      : 2 * waves;
         auto o_size = [&](long long n) {

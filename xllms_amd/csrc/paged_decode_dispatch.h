@@ -66,34 +66,51 @@ static hipError_t launch_partition(F kernel, unsigned grid, unsigned block, size
 
 template <int KV, int D, int GT, int TT>
 static hipError_t launch_merge(const DecodeParams &p, hipStream_t st) {
-    const unsigned segs = (unsigned)(p.num_seqs * p.num_kv_heads * p.head_tiles);
+    const unsigned segs = (unsigned)(p.num_kv_heads * p.head_tiles);
     const int heads = p.group < GT ? p.group : GT;
+    const int cols = heads * (D / 4);
     if (p.merge_per_segment) {
         // one thread per float4 column of the segment (heads * D/4), the
-        // count rounded up to a power of two from 64 to 1024; the wider
-        // instantiations exist only where a segment can have that many
-        // columns (fewer than 64 columns: 64 threads split the partials)
+        // count rounded up to a power of two from 64 to 1024; up to 32
+        // columns, the lanes of one wavefront share them.  Instantiations
+        // exist only where a segment can have that many columns.
+        const dim3 grid(segs, (unsigned)p.num_seqs);
         constexpr int kMaxCols = GT * (D / 4);
         constexpr int kNt128 = kMaxCols > 64 ? 128 : 64;
         constexpr int kNt256 = kMaxCols > 128 ? 256 : 64;
         constexpr int kNt512 = kMaxCols > 256 ? 512 : 64;
         constexpr int kNt1024 = kMaxCols > 512 ? 1024 : 64;
-        const int cols = heads * (D / 4);
-        if (cols <= 64)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, 64><<<segs, 64, 0, st>>>(p);
+        if (cols <= 8)
+            paged_decode_merge_segment_kernel<KV, D, GT, TT, 64, 8><<<grid, 64, 0, st>>>(p);
+        else if (cols <= 16)
+            paged_decode_merge_segment_kernel<KV, D, GT, TT, 64, 4><<<grid, 64, 0, st>>>(p);
+        else if (cols <= 32)
+            paged_decode_merge_segment_kernel<KV, D, GT, TT, 64, 2><<<grid, 64, 0, st>>>(p);
+        else if (cols <= 64)
+            paged_decode_merge_segment_kernel<KV, D, GT, TT, 64, 1><<<grid, 64, 0, st>>>(p);
         else if (cols <= 128)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt128><<<segs, kNt128, 0, st>>>(p);
+            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt128, 1><<<grid, kNt128, 0, st>>>(p);
         else if (cols <= 256)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt256><<<segs, kNt256, 0, st>>>(p);
+            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt256, 1><<<grid, kNt256, 0, st>>>(p);
         else if (cols <= 512)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt512><<<segs, kNt512, 0, st>>>(p);
+            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt512, 1><<<grid, kNt512, 0, st>>>(p);
         else
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt1024><<<segs, kNt1024, 0, st>>>(p);
+            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt1024, 1>
+                <<<grid, kNt1024, 0, st>>>(p);
         return hipGetLastError();
     }
-    const unsigned chunks = (unsigned)((heads * (D / 4) + kMergeCols - 1) / kMergeCols);
-    paged_decode_merge_kernel<KV, D, GT, TT>
-        <<<dim3(segs, chunks), kMergeCols * kMergeSplit, 0, st>>>(p);
+    const dim3 grid(segs, (unsigned)((cols + kMergeCols - 1) / kMergeCols), (unsigned)p.num_seqs);
+    // the new-token fold needs a head's columns in one aligned lane group
+    constexpr bool kFold = D == 32 || D == 64 || D == 128;
+    if constexpr (kFold) {
+        if (p.nt_fold) {
+            paged_decode_merge_kernel<KV, D, GT, TT, true>
+                <<<grid, kMergeCols * kMergeSplit, 0, st>>>(p);
+            return hipGetLastError();
+        }
+    }
+    paged_decode_merge_kernel<KV, D, GT, TT, false>
+        <<<grid, kMergeCols * kMergeSplit, 0, st>>>(p);
     return hipGetLastError();
 }
 

@@ -541,6 +541,7 @@ __device__ __forceinline__ void stream_k_walk(const DecodeParams &p, int *pre, F
     const int total = pre[B];
     const int w = logical_block(p, total) * WPG + wave;
     const int tpw = tiles_per_wave(total, p.num_waves, p.min_tiles_per_wave);
+    if (blockIdx.x == 0 && threadIdx.x == 0) p.ws_prefix[B + 1] = tpw;
     const long long g_lo = (long long)w * tpw;
     if (g_lo >= total) return;
     int g = (int)g_lo;
@@ -890,7 +891,7 @@ __global__ __launch_bounds__(256) void paged_decode_segment_merge_kernel(const D
 // The slots of a cut segment's partials: partial 0 in slot s0, partial
 // j >= 1 in slot sb + sstride * j.
 struct PartialSlots {
-    size_t s0, sb;
+    int s0, sb;
     int sstride, np;
 };
 
@@ -907,17 +908,17 @@ __device__ __forceinline__ bool segment_partials(const DecodeParams &p, int seg_
     // the segment is w_first's first piece when w_first's range begins in the
     // segment's start-up units or at its first tile
     const int slot0 = (w_first * tpw >= seg_start) ? 0 : 1;
-    ps.s0 = (size_t)w_first * 2 + slot0;
+    ps.s0 = w_first * 2 + slot0;
     if (p.wg_fix) {
         const int wg0 = w_first / WPG, wg1 = w_last / WPG;
         if (wg0 == wg1) return false;
         ps.np = wg1 - wg0 + 1;
-        ps.sb = (size_t)wg0 * 2 * WPG;
+        ps.sb = wg0 * 2 * WPG;
         ps.sstride = 2 * WPG;
     } else {
         if (w_first == w_last) return false;
         ps.np = w_last - w_first + 1;
-        ps.sb = (size_t)w_first * 2;
+        ps.sb = w_first * 2;
         ps.sstride = 2;
     }
     return true;
@@ -933,7 +934,7 @@ __device__ __forceinline__ bool segment_partials_paired(int seg_start, int first
     if (r_first == r_last) return false;
     const int slot0 = (r_first * tpw >= seg_start) ? 0 : 1;
     ps.np = r_last - r_first + 1;
-    ps.sb = (size_t)(2 * r_first + ht) * 2;
+    ps.sb = (2 * r_first + ht) * 2;
     ps.s0 = ps.sb + slot0;
     ps.sstride = 4;
     return true;
@@ -957,15 +958,19 @@ __device__ __forceinline__ f32x4 partial_f32x4(const DecodeParams &p, size_t at)
 // segment's partials j = j0, j0 + step, ... < np (slots as in PartialSlots).
 // The partials go in batches of up to NB whose loads are all issued before
 // any is used, so a thread waits for one memory round trip per batch, not
-// per partial; batch slots past np load and combine nothing.  The column's
-// (m, l) and float4 of o sit at off_ml and off_o floats into a slot.  HS:
-// fp16 states (DecodeParams::ws_h), whose o is read at the same index.
+// per partial; batch slots past np load and combine nothing.  A batch is
+// combined under its largest running max: one exponential and five
+// multiply-adds per partial.  The column's (m, l) and float4 of o sit at
+// off_ml and off_o floats into a slot.  HS: fp16 states (DecodeParams::ws_h),
+// whose o is read at the same index.
 template <int GT, int D, int NB, bool HS = false>
 __device__ __forceinline__ void merge_partials(const DecodeParams &p, const PartialSlots &ps,
                                                int j0, int step, int off_ml, int off_o,
                                                float &m, float &l, f32x4 &acc) {
-    const int np = ps.np;
-    for (int jb = j0; jb < np; jb += NB * step) {
+    const float *ml = p.ws_ml + off_ml;
+    const char *o = HS ? (const char *)p.ws_h + (size_t)off_o * 2 : (const char *)(p.ws_o + off_o);
+#pragma unroll 1
+    for (int jb = j0; jb < ps.np; jb += NB * step) {
         f32x2 mlv[NB];
         f32x4 ov[NB];
         u32x2 hv[NB];
@@ -975,56 +980,67 @@ __device__ __forceinline__ void merge_partials(const DecodeParams &p, const Part
             mlv[b] = f32x2{-INFINITY, 0.0f};  // (defined values for the slots left unread)
             ov[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             hv[b] = u32x2{0u, 0u};
-            if (j < np) {
-                const size_t slot = j == 0 ? ps.s0 : ps.sb + (size_t)ps.sstride * j;
-                mlv[b] = *(const f32x2 *)(p.ws_ml + slot * GT * 2 + off_ml);
-                if constexpr (HS)
-                    hv[b] = *(const u32x2 *)((const char *)p.ws_h + (slot * GT * D + off_o) * 2);
-                else
-                    ov[b] = *(const f32x4 *)(p.ws_o + slot * GT * D + off_o);
+            if (j < ps.np) {
+                const size_t slot = (uint32_t)(j == 0 ? ps.s0 : ps.sb + ps.sstride * j);
+                mlv[b] = *(const f32x2 *)(ml + slot * (GT * 2));
+                if constexpr (HS) hv[b] = *(const u32x2 *)(o + slot * (GT * D * 2));
+                else ov[b] = *(const f32x4 *)(o + slot * (GT * D * 4));
             }
         }
         // keep the scheduler from starting the combine (and waiting on the
         // first loads) before the whole batch is issued
         __builtin_amdgcn_sched_barrier(0);
+        float M = m;
+#pragma unroll
+        for (int b = 0; b < NB; b++) M = fmaxf(M, mlv[b].x);
+        const float Ms = (M == -INFINITY) ? 0.0f : M;
+        const float a = fast_exp2(m - Ms);
+        l *= a;
+        acc *= a;
 #pragma unroll
         for (int b = 0; b < NB; b++) {
-            if (jb + b * step >= np) break;
             if constexpr (HS) ov[b] = unpack_h4(hv[b]);
-            const float mj = mlv[b].x;
-            const float M = fmaxf(m, mj);
-            const float Ms = (M == -INFINITY) ? 0.0f : M;
-            const float a = fast_exp2(m - Ms), w = fast_exp2(mj - Ms);
-            l = l * a + mlv[b].y * w;
-            acc = acc * a + ov[b] * w;
-            m = M;
+            const float w = fast_exp2(mlv[b].x - Ms);
+            l = fmaf(mlv[b].y, w, l);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[e] = fmaf(ov[b][e], w, acc[e]);
         }
+        m = M;
     }
 }
 
-// Output float4 column `col` (head col / (D/4), head-major) of an empty
-// sequence s: zeros (log-sum-exp -inf), or the prefix row under a prefix
-// fold (the sequence's whole context was the shared prefix).
-template <int KV, int D>
-__device__ __forceinline__ void write_empty_column(const DecodeParams &p, int s, int kvh, int g0,
-                                                   size_t qrow0, int col) {
-    constexpr int C4 = D / 4;
-    const size_t base = qrow0 + (size_t)col * 4;
-    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-    float lse = -INFINITY;
+// State of a column (head h of the tile, float4 c) of an empty sequence s:
+// nothing, or the prefix row under a prefix fold (the sequence's whole
+// context was the shared prefix).
+template <int D>
+__device__ __forceinline__ void empty_state(const DecodeParams &p, int s, int kvh, int head, int c,
+                                            float &m, float &l, f32x4 &acc) {
     const int fb = p.fold_row ? p.fold_row[s] : -1;
-    if (fb >= 0) {
-        const size_t r = fold_state_row(p, fb, kvh, g0 + col / C4);
-        o = *(const f32x4 *)(p.fold_out + r * D + (col % C4) * 4);
-        lse = p.fold_lse[r];
-    }
+    if (fb < 0) return;
+    const size_t r = fold_state_row(p, fb, kvh, head);
+    m = p.fold_lse[r];
+    l = 1.0f;
+    acc = *(const f32x4 *)(p.fold_out + r * D + c * 4);
+}
+
+// Four consecutive elements, from element i of an output row.
+template <int KV> __device__ __forceinline__ void store4(char *row, int i, f32x4 o) {
+    if constexpr (KV == KV_F32) *(f32x4 *)(row + (size_t)i * 4) = o;
+    else *(u32x2 *)(row + (size_t)i * 2) = u32x2{pack16<KV>(o[0], o[1]), pack16<KV>(o[2], o[3])};
+}
+
+// The finished column (head h of the tile, float4 c) of a state: its output,
+// or in partial-output mode its fp32 row and log-sum-exp.
+template <int KV, int D>
+__device__ __forceinline__ void write_column(const DecodeParams &p, int s, int head, int c, float m,
+                                             float l, f32x4 acc) {
+    const f32x4 o = acc * (l > 0.0f ? 1.0f / l : 0.0f);
     if (p.out_f32) {
-        *(f32x4 *)(p.out_f32 + base) = o;
-        if (col % C4 == 0) p.out_lse[qrow0 / D + col / C4] = lse;
+        const size_t row = (size_t)s * p.num_heads + head;
+        *(f32x4 *)(p.out_f32 + row * D + c * 4) = o;
+        if (c == 0) p.out_lse[row] = l > 0.0f ? m + log2f(l) : -INFINITY;
     } else {
-        char *orow = o_row(p, s, kvh * p.group + g0 + col / C4, D, KV == KV_F32 ? 4 : 2);
-#pragma unroll
-        for (int e = 0; e < 4; e++) store_elem<KV>(orow, (col % C4) * 4 + e, o[e]);
+        store4<KV>(o_row(p, s, head, D, KV == KV_F32 ? 4 : 2), c * 4, o);
     }
 }
 
@@ -1101,250 +1117,174 @@ __device__ __forceinline__ void store_new_token(const DecodeParams &p, int kvh, 
     }
 }
 
+// The merge launches are short chains -- lengths and ranges, then partials --
+// of a few hundred workgroups whose instructions come from a cold cache at
+// every launch: their time follows the code they run through.  So a launch
+// gets only what it needs: the new-token fold and the split of a column's
+// partials are template arguments, the grid's dimensions name the segment,
+// and the partition kernel hands over its units per wavefront
+// (ws_prefix[num_seqs + 1]).  At 2.9-3.7 KB each instead of 5.4-8 KB a step
+// takes 0.5-0.9 us less (fp16, 32 / 8 heads: 16 x 1024 tokens 20.8 -> 20.0
+// us, 4 sequences of 8192-32768 60.8 -> 59.9, head_size 80, 32 heads, 24 of
+// 100-2000 50.7 -> 49.9); 2 KB more of range arithmetic in them cost 1.1 us.
+
 // Merge kernel: one workgroup per (segment, chunk of kMergeCols output
-// float4 columns), where a segment is (sequence, kv head, head tile) and the
+// float4 columns, sequence), where a segment is (kv head, head tile) and the
 // columns run over (head h < nh, dims 4c..4c+3).  It writes zeros for an
 // empty sequence, does nothing for a segment finished inside one wavefront
 // range, and otherwise combines the partials of every wavefront that touched
-// the segment in one pass: each of the kMergeSplit threads of a column runs
-// an online log-sum-exp merge over every kMergeSplit-th partial (running max,
-// rescaled denominator and float4 numerator), and the splits are combined in
-// LDS the same way.  TT is the tile length (tokens) of the partition kernel
-// that produced the partials: the range arithmetic must match it exactly.
+// the segment: each of the kMergeSplit threads of a column merges every
+// kMergeSplit-th partial, and the splits are combined in LDS.  TT is the
+// tile length (tokens) of the partition kernel that produced the partials:
+// the range arithmetic must match it exactly.  NTF: the new-token fold
+// (DecodeParams::nt_fold).
 constexpr int kMergeSplit = 8;
 
-template <int KV, int D, int GT, int TT>
+template <int KV, int D, int GT, int TT, bool NTF>
 __global__ __launch_bounds__(kMergeCols * kMergeSplit) void paged_decode_merge_kernel(
     const DecodeParams p) {
     XHIP_MERGE_SCOPE(p);
     constexpr int C4 = D / 4;
+    constexpr int EB = KV == KV_F32 ? 4 : 2;
     __shared__ f32x4 s_acc[kMergeSplit][kMergeCols];
     __shared__ float s_m[kMergeSplit][kMergeCols];
     __shared__ float s_l[kMergeSplit][kMergeCols];
-    const int segs = p.num_kv_heads * p.head_tiles;
-    const int s = blockIdx.x / segs;
-    const int seg = blockIdx.x - s * segs;
-    const int kvh = seg / p.head_tiles;
-    const int ht = seg - kvh * p.head_tiles;
-    const int g0 = ht * GT;
-    const int nh = min(GT, p.group - g0);
-    const int ncols = nh * C4;
-    const int col0 = blockIdx.y * kMergeCols;
-    constexpr int EB = KV == KV_F32 ? 4 : 2;
-    // the new-token fold needs a head's columns in one aligned lane group
-    constexpr bool kFold = (C4 & (C4 - 1)) == 0 && C4 <= 32;
-    if (kFold && p.nt_fold && blockIdx.y == 0 && ht == 0)
-        store_new_token<D, EB>(p, kvh, blockIdx.x == 0);
-    if (col0 >= ncols) return;
-    const int tid = threadIdx.x;
-    // the new-token fold's threads: the first kMergeCols, one per column
-    FoldIn fi;
-    if constexpr (kFold) {
-        if (p.nt_fold && tid < kMergeCols && col0 + tid < ncols) {
-            const int h = (col0 + tid) / C4;
-            fi = fold_load<KV, D>(p, s, kvh, kvh * p.group + g0 + h, col0 + tid - h * C4);
-        }
-    }
-    // the three scalars the merge needs, requested together (the empty asm
-    // keeps the compiler from sinking the prefix loads past the L == 0 exit,
-    // which would cost a second round trip).  Under the new-token fold (one
-    // sequence, its cached length by value) they need no load at all.
+    const int s = blockIdx.z, seg = blockIdx.x;
+    // the scalars the merge needs, requested together (the empty asm keeps
+    // the compiler from sinking loads past the L == 0 branch, which would
+    // cost a second round trip).  Under the new-token fold (one sequence, its
+    // cached length by value) they need no load at all.
     const int L = seq_len_of(p, s);
-    int total, pre_s;
-    if (kFold && p.nt_fold) {
-        total = segs * segment_units(p, (L + TT - 1) / TT);
-        pre_s = 0;
+    int tpw, pre_s = 0;
+    if constexpr (NTF) {
+        tpw = tiles_per_wave(gridDim.x * segment_units(p, (L + TT - 1) / TT), p.num_waves,
+                             p.min_tiles_per_wave);
     } else {
-        total = p.ws_prefix[p.num_seqs];
+        tpw = p.ws_prefix[p.num_seqs + 1];
         pre_s = p.ws_prefix[s];
+        asm volatile("" ::"s"(tpw), "s"(pre_s));
     }
-    asm volatile("" ::"s"(total), "s"(pre_s));
-    const size_t qrow0 = ((size_t)s * p.num_heads + (size_t)kvh * p.group + g0) * D;
+    int kvh = seg, g0 = 0;
+    if (p.head_tiles != 1) {
+        kvh = seg / p.head_tiles;
+        g0 = (seg - kvh * p.head_tiles) * GT;
+    }
+    const int tid = threadIdx.x;
+    const int cl = tid % kMergeCols;
+    const int psplit = tid / kMergeCols;
+    const int col = blockIdx.y * kMergeCols + cl;
+    if (NTF && blockIdx.y == 0 && g0 == 0) store_new_token<D, EB>(p, kvh, seg == 0);
+    const bool active = col < min(GT, p.group - g0) * C4;
+    const int h = col / C4, c = col - h * C4;
+    const int head = kvh * p.group + g0 + h;
+    const bool writer = active && psplit == 0;
+    FoldIn fi;
+    if constexpr (NTF)
+        if (writer) fi = fold_load<KV, D>(p, s, kvh, head, c);
 
-    if (L == 0) {
-        if constexpr (kFold) {
-            if (p.nt_fold) {  // no cached token: the output is the new token's V
-                const int col = col0 + tid;
-                if (tid < kMergeCols && col < ncols) {
-                    const int h = col / C4, c = col - h * C4;
-                    const f32x4 o = fold_new_token<D>(p, fi, -INFINITY, 0.0f,
-                                                      f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-                    char *orow = o_row(p, s, kvh * p.group + g0 + h, D, EB);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) store_elem<KV>(orow, c * 4 + e, o[e]);
-                }
-                return;
-            }
-        }
-        if (tid < kMergeCols && col0 + tid < ncols && !p.skip_empty)
-            write_empty_column<KV, D>(p, s, kvh, g0, qrow0, col0 + tid);
-        return;
-    }
-    const int tpw = tiles_per_wave(total, p.num_waves, p.min_tiles_per_wave);
+    float m = -INFINITY, l = 0.0f;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     const int Ts = (L + TT - 1) / TT;
     const int seg_start = pre_s + seg * segment_units(p, Ts);  // in split units
     PartialSlots ps;
-    if (!segment_partials<kMfmaWavesPerGroup>(p, seg_start, seg_start + p.seg_cost, Ts, tpw, ps)) {
-        if constexpr (kFold) {
-            if (p.nt_fold) {
-                // a segment the partition kernel finished: its row and
-                // log-sum-exp (partial-output mode), folded with the new token
-                const int col = col0 + tid;
-                if (tid < kMergeCols && col < ncols) {
-                    const int h = col / C4, c = col - h * C4;
-                    const float lse = p.out_lse[qrow0 / D + h];
-                    const f32x4 row = *(const f32x4 *)(p.out_f32 + qrow0 + (size_t)h * D + c * 4);
-                    const f32x4 o =
-                        fold_new_token<D>(p, fi, lse, lse == -INFINITY ? 0.0f : 1.0f, row);
-                    char *orow = o_row(p, s, kvh * p.group + g0 + h, D, EB);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) store_elem<KV>(orow, c * 4 + e, o[e]);
-                }
-            }
+    if (L == 0) {
+        if (!NTF && p.skip_empty) return;
+        if (!NTF && writer) empty_state<D>(p, s, kvh, g0 + h, c, m, l, acc);
+    } else if (!segment_partials<kMfmaWavesPerGroup>(p, seg_start, seg_start + p.seg_cost, Ts, tpw,
+                                                     ps)) {
+        if (!NTF) return;
+        if (writer) {
+            // a segment the partition kernel finished: its row and
+            // log-sum-exp (partial-output mode)
+            const size_t row = (size_t)s * p.num_heads + head;
+            m = p.out_lse[row];
+            l = m == -INFINITY ? 0.0f : 1.0f;
+            acc = *(const f32x4 *)(p.out_f32 + row * D + c * 4);
         }
-        return;
-    }
-
-    const int cl = tid % kMergeCols;
-    const int psplit = tid / kMergeCols;
-    const int col = col0 + cl;
-    const bool active = col < ncols;
-    const int h = active ? col / C4 : 0;
-    const int c = active ? col - h * C4 : 0;
-    float m = -INFINITY, l = 0.0f;
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (active) merge_partials<GT, D, 8>(p, ps, psplit, kMergeSplit, h * 2, h * D + c * 4, m, l, acc);
-    s_acc[psplit][cl] = acc;
-    s_m[psplit][cl] = m;
-    s_l[psplit][cl] = l;
-    __syncthreads();
-    if (psplit != 0 || !active) return;
-    float mm = m, ll = l;
-    f32x4 aa = acc;
+    } else {
+        if (active)
+            merge_partials<GT, D, 8>(p, ps, psplit, kMergeSplit, h * 2, h * D + c * 4, m, l, acc);
+        s_acc[psplit][cl] = acc;
+        s_m[psplit][cl] = m;
+        s_l[psplit][cl] = l;
+        __syncthreads();
+        if (!writer) return;
 #pragma unroll
-    for (int k = 1; k < kMergeSplit; k++) {
-        const float mk = s_m[k][cl];
-        const float M = fmaxf(mm, mk);
-        const float Ms = (M == -INFINITY) ? 0.0f : M;
-        const float a = fast_exp2(mm - Ms), b = fast_exp2(mk - Ms);
-        ll = ll * a + s_l[k][cl] * b;
-        aa = aa * a + s_acc[k][cl] * b;
-        mm = M;
-    }
-    if constexpr (kFold) {
-        if (p.nt_fold) {
-            const f32x4 o = fold_new_token<D>(p, fi, mm, ll, aa);
-            char *orow = o_row(p, s, kvh * p.group + g0 + h, D, EB);
+        for (int k = 1; k < kMergeSplit; k++) m = fmaxf(m, s_m[k][cl]);
+        const float Ms = (m == -INFINITY) ? 0.0f : m;
+        l = 0.0f;
+        acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int e = 0; e < 4; e++) store_elem<KV>(orow, c * 4 + e, o[e]);
-            return;
+        for (int k = 0; k < kMergeSplit; k++) {
+            const float w = fast_exp2(s_m[k][cl] - Ms);
+            const f32x4 o = s_acc[k][cl];
+            l = fmaf(s_l[k][cl], w, l);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[e] = fmaf(o[e], w, acc[e]);
         }
     }
-    const float inv = ll > 0.0f ? 1.0f / ll : 0.0f;
-    const size_t base = qrow0 + (size_t)h * D + c * 4;
-    if (p.out_f32) {
-        *(f32x4 *)(p.out_f32 + base) = aa * inv;
-        if (c == 0) p.out_lse[qrow0 / D + h] = ll > 0.0f ? mm + log2f(ll) : -INFINITY;
-        return;
-    }
-    char *orow = o_row(p, s, kvh * p.group + g0 + h, D, EB);
-#pragma unroll
-    for (int e = 0; e < 4; e++) store_elem<KV>(orow, c * 4 + e, aa[e] * inv);
+    if (!writer) return;
+    if constexpr (NTF)
+        store4<KV>(o_row(p, s, head, D, EB), c * 4, fold_new_token<D>(p, fi, m, l, acc));
+    else
+        write_column<KV, D>(p, s, head, c, m, l, acc);
 }
 
-
-// Merge kernel, one workgroup per segment: for batches with enough segments
-// to fill the GPU (where the (segment, chunk) grid above would launch several
+// Merge kernel, one workgroup per (segment, sequence): for batches with
+// enough segments to fill the GPU (where the grid above would launch several
 // thousand short workgroups, each costing ~2 ns of dispatch).  NT threads
 // (64 to 1024, chosen at launch as the first head tile's float4 columns
 // rounded up to a power of two, at least 64) cover the columns, one each;
-// where a segment has at most NT / 2 columns (fewer than 64, or the partly
-// filled last head tile of a group), the S = NT / pow2(ncols) threads of a
-// column split its partials (every S-th one) and combine in LDS.  Each thread runs
-// the online log-sum-exp merge over its partials with a batch of their loads
-// in flight at a time.
-constexpr int kMergeSegThreads = 64;  // the smallest NT (LDS split below that many columns)
-
-template <int KV, int D, int GT, int TT, int NT>
+// with fewer than 64 columns, SPL = 64 / pow2(columns) lanes of the one
+// wavefront share a column, each merging every SPL-th partial.
+template <int KV, int D, int GT, int TT, int NT, int SPL>
 __global__ __launch_bounds__(NT) void paged_decode_merge_segment_kernel(const DecodeParams p) {
     XHIP_MERGE_SCOPE(p);
+    static_assert(SPL == 1 || NT == 64, "the lanes of a column are in one wavefront");
     constexpr int C4 = D / 4;
-    __shared__ f32x4 s_acc[NT];
-    __shared__ float s_m[NT];
-    __shared__ float s_l[NT];
-    const int segs = p.num_kv_heads * p.head_tiles;
-    const int s = blockIdx.x / segs;
-    const int seg = blockIdx.x - s * segs;
-    const int kvh = seg / p.head_tiles;
-    const int g0 = (seg - kvh * p.head_tiles) * GT;
-    const int nh = min(GT, p.group - g0);
-    const int ncols = nh * C4;
-    // a head tile with no heads has nothing to merge (the host never plans
-    // one; the column-span loop below needs ncols >= 1 to end)
-    if (ncols <= 0) return;
-    const int tid = threadIdx.x;
-    // the three scalars the merge needs, requested together (the empty asm
-    // keeps the compiler from sinking the prefix loads past the L == 0 exit,
-    // which would cost a second round trip)
+    constexpr int kSpan = NT / SPL;
+    const int s = blockIdx.y, seg = blockIdx.x;
+    // the scalars the merge needs, requested together (as above)
     const int L = seq_len_of(p, s);
-    const int total = p.ws_prefix[p.num_seqs];
+    const int tpw = p.ws_prefix[p.num_seqs + 1];
     const int pre_s = p.ws_prefix[s];
-    asm volatile("" ::"s"(total), "s"(pre_s));
-    const size_t qrow0 = ((size_t)s * p.num_heads + (size_t)kvh * p.group + g0) * D;
-
-    if (L == 0) {
-        if (!p.skip_empty)
-            for (int col = tid; col < ncols; col += NT) write_empty_column<KV, D>(p, s, kvh, g0, qrow0, col);
-        return;
+    asm volatile("" ::"s"(tpw), "s"(pre_s));
+    int kvh = seg, g0 = 0;
+    if (p.head_tiles != 1) {
+        kvh = seg / p.head_tiles;
+        g0 = (seg - kvh * p.head_tiles) * GT;
     }
-    const int tpw = tiles_per_wave(total, p.num_waves, p.min_tiles_per_wave);
-    const int Ts = (L + TT - 1) / TT;
-    const int seg_start = pre_s + seg * segment_units(p, Ts);  // in split units
-    PartialSlots ps;
-    if (!segment_partials<kMfmaWavesPerGroup>(p, seg_start, seg_start + p.seg_cost, Ts, tpw, ps))
-        return;
-
-    // Column span per split: all NT threads when ncols > NT / 2, else pow2(ncols).
-    int span = NT;
-    while ((span >> 1) >= ncols) span >>= 1;
-    const int split = tid / span;  // 0 .. S-1
-    const int nsplit = NT / span;
-    const int cl = tid - split * span;
+    const int cl = threadIdx.x % kSpan;
+    const int split = threadIdx.x / kSpan;  // (0 with SPL == 1)
+    if (cl >= min(GT, p.group - g0) * C4) return;
+    const int h = cl / C4, c = cl - h * C4;
 
     float m = -INFINITY, l = 0.0f;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (cl < ncols) {
-        const int h = cl / C4;
-        merge_partials<GT, D, 8>(p, ps, split, nsplit, h * 2, h * D + (cl - h * C4) * 4, m, l, acc);
-    }
-    if (nsplit > 1) {  // ncols <= NT / 2: fewer than 64 columns, or a partly filled last head tile
-        s_acc[tid] = acc;
-        s_m[tid] = m;
-        s_l[tid] = l;
-        __syncthreads();
-        if (split != 0) return;
-        for (int k = 1; k < nsplit; k++) {
-            const int o = k * span + cl;
-            const float mk = s_m[o];
-            const float M = fmaxf(m, mk);
+    if (L == 0) {
+        if (p.skip_empty) return;
+        empty_state<D>(p, s, kvh, g0 + h, c, m, l, acc);
+    } else {
+        const int Ts = (L + TT - 1) / TT;
+        const int seg_start = pre_s + seg * segment_units(p, Ts);  // in split units
+        PartialSlots ps;
+        if (!segment_partials<kMfmaWavesPerGroup>(p, seg_start, seg_start + p.seg_cost, Ts, tpw,
+                                                  ps))
+            return;
+        merge_partials<GT, D, 8>(p, ps, SPL == 1 ? 0 : split, SPL, h * 2, h * D + c * 4, m, l, acc);
+#pragma unroll
+        for (int off = kSpan; off < NT && SPL > 1; off <<= 1) {
+            const float mo = __shfl_xor(m, off);
+            const float M = fmaxf(m, mo);
             const float Ms = (M == -INFINITY) ? 0.0f : M;
-            const float a = fast_exp2(m - Ms), b = fast_exp2(mk - Ms);
-            l = l * a + s_l[o] * b;
-            acc = acc * a + s_acc[o] * b;
+            const float a = fast_exp2(m - Ms), b = fast_exp2(mo - Ms);
+            l = l * a + __shfl_xor(l, off) * b;
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[e] = acc[e] * a + __shfl_xor(acc[e], off) * b;
             m = M;
         }
     }
-    if (cl >= ncols) return;
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    const size_t base = qrow0 + (size_t)cl * 4;  // head-major columns
-    if (p.out_f32) {
-        *(f32x4 *)(p.out_f32 + base) = acc * inv;
-        if (cl % C4 == 0) p.out_lse[qrow0 / D + cl / C4] = l > 0.0f ? m + log2f(l) : -INFINITY;
-        return;
-    }
-    char *orow = o_row(p, s, kvh * p.group + g0 + cl / C4, D, KV == KV_F32 ? 4 : 2);
-#pragma unroll
-    for (int e = 0; e < 4; e++) store_elem<KV>(orow, (cl % C4) * 4 + e, acc[e] * inv);
+    if (split == 0) write_column<KV, D>(p, s, kvh * p.group + g0 + h, c, m, l, acc);
 }
 
 }  // namespace xhip

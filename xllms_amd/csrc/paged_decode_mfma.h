@@ -1193,6 +1193,9 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, D <= 128 ? 2 : 1) void pag
     const int lb = logical_block(p, pre[p.num_seqs]);
     XHIP_WG_PUT(p, 3, lb);
     mfma_partition_body<KV, D, R>(p, lens, tables, pre, lb, p.num_waves, sm);
+    if (blockIdx.x == 0 && threadIdx.x == 0)  // for the merge
+        p.ws_prefix[p.num_seqs + 1] =
+            tiles_per_wave(pre[p.num_seqs], p.num_waves, p.min_tiles_per_wave);
     XHIP_WG_FLUSH(p);
 }
 

@@ -93,7 +93,9 @@ __device__ __forceinline__ unsigned long long *wg_trace_lds() {
         unsigned long long t0_;                                                                \
         __device__ ~XhipMergeExit_() {                                                         \
             const unsigned long long b_ = (unsigned long long)blockIdx.x +                     \
-                                          (unsigned long long)blockIdx.y * gridDim.x;          \
+                                          (unsigned long long)gridDim.x *                  \
+                                              (blockIdx.y + (unsigned long long)gridDim.y *    \
+                                                                blockIdx.z);                   \
             if (p_.wg_trace && threadIdx.x == 0 && b_ < ::xhip::kWgTraceMergeMax) {            \
                 p_.wg_trace[::xhip::kWgTraceMergeBase + 2 * b_] = t0_;                         \
                 p_.wg_trace[::xhip::kWgTraceMergeBase + 2 * b_ + 1] =                          \
