@@ -36,3 +36,33 @@ def test_tile_edges(cuda, dtype, head_size, group):
                           kv_dtype=DT[dtype], seed=head_size + group + bs, lens=lens)
         print(f"case {dtype} d={head_size} group={group} bs={bs}", flush=True)
         _check(wl, f"{dtype} d={head_size} group={group} bs={bs}")
+
+
+@pytest.mark.parametrize("head_size", [32, 64, 96, 128])
+@pytest.mark.parametrize("group", [5, 8, 16, 17, 32])
+def test_fp32_tile_edges(cuda, head_size, group):
+    """fp32 automatic plans take the matrix tiles for groups above 4 at any
+    length: edges of the 16-token tile, one and two head tiles, pages of one
+    and two tiles."""
+    lens = [1, 2, 3, 4, 5, 15, 16, 17, 31, 32, 33, 0, 255, 1025]
+    for bs in (16, 32):
+        wl = W.small_case(num_seqs=len(lens), H=2 * group, KVH=2, D=head_size, bs=bs,
+                          kv_dtype=W.FP32, seed=head_size + group + bs, lens=lens)
+        print(f"case fp32 d={head_size} group={group} bs={bs}", flush=True)
+        _check(wl, f"fp32 d={head_size} group={group} bs={bs}")
+
+
+@pytest.mark.parametrize("case", [
+    # (H, KVH, seqs, tokens): fp32, head_size 128, batches just below and
+    # above the K/V bytes from which groups of up to 4 (32 MB) and up to 2
+    # (128 MB) take the matrix tiles; 33 kv heads x 8 sequences are more
+    # segments than CUs (no segment launch)
+    (8, 2, 15, 1024), (8, 2, 16, 1024), (33, 33, 8, 464), (33, 33, 8, 480), (34, 17, 16, 448),
+    (34, 17, 16, 480),
+])
+def test_fp32_tile_path_rule(cuda, case):
+    H, KVH, n, tokens = case
+    lens = [max(1, tokens - 67 * i) for i in range(n)]
+    wl = W.small_case(num_seqs=n, H=H, KVH=KVH, D=128, kv_dtype=W.FP32, seed=n + tokens, lens=lens)
+    print(f"case H={H} KVH={KVH} seqs={n} tokens={tokens}", flush=True)
+    _check(wl, f"H={H} KVH={KVH} seqs={n} tokens={tokens}")

@@ -181,6 +181,15 @@ bool use_mfma(int kv_dtype, int head_size, int block_size) {
     return kv_dtype != NXT_KV_FP32 && head_size % 32 == 0 && block_size >= 16;
 }
 
+// Shapes outside use_mfma whose automatic stream-K plans may take the MFMA
+// tiles (auto_mfma): fp32 at head sizes whose tiles fit the registers.
+// Explicit partition_tokens plans keep the VALU tile, whose length is their
+// unit.
+bool use_mfma_auto(int kv_dtype, int head_size, int block_size) {
+    return kv_dtype == NXT_KV_FP32 && head_size % 32 == 0 &&
+           head_size <= xhip::kMfmaF32MaxHeadSize && block_size >= 16;
+}
+
 // Tokens per tile of the kernel instantiation: 16 on the MFMA path, else
 // kLoadsPerTile loads of 64/lanes-per-row rows (mirrors xhip::Geometry).
 int tile_tokens(int head_size, int kv_dtype, bool mfma) {
@@ -201,13 +210,14 @@ int max_group(bool mfma) {
     return mfma ? xhip::kMfmaMaxGroup : xhip::kMaxHeadTile * xhip::kWavesPerGroup;
 }
 
-bool head_tiling(int group, bool mfma, int head_size, HeadTiling *t) {
+bool head_tiling(int group, bool mfma, int kv_dtype, int head_size, HeadTiling *t) {
     if (group <= 0 || group > max_group(mfma)) return false;
     if (mfma) {
         // groups of 17-32 heads: one wavefront with two row blocks reads each
-        // K/V tile once for all of them (head_size <= 128), else two
-        // wavefronts of one block each
-        const bool wide = group > xhip::kMfmaHeads && head_size <= xhip::kMfmaWideMaxHeadSize;
+        // K/V tile once for all of them (16-bit types, head_size <= 128),
+        // else two wavefronts of one block each
+        const bool wide = group > xhip::kMfmaHeads && kv_dtype != NXT_KV_FP32 &&
+                          head_size <= xhip::kMfmaWideMaxHeadSize;
         t->head_tile = wide ? 2 * xhip::kMfmaHeads : xhip::kMfmaHeads;
         t->head_tiles = (group + t->head_tile - 1) / t->head_tile;
         return true;
@@ -222,6 +232,32 @@ bool head_tiling(int group, bool mfma, int head_size, HeadTiling *t) {
     t->head_tile = xhip::kMaxHeadTile;
     t->head_tiles = (group + xhip::kMaxHeadTile - 1) / xhip::kMaxHeadTile;
     return t->head_tiles <= xhip::kWavesPerGroup;
+}
+
+// Small batches on the VALU tile path: one round of workgroups over the
+// segments (paged_decode_segment_kernel) when they fit one per CU, S of them
+// per segment.  A workgroup streams its share of a segment through one CU
+// (~68 GB/s measured on MI355X), so a segment is split while each share keeps
+// at least kSegSplitBytes of K/V, which one CU streams in about the time the
+// merge launch then needed takes (~2.3 us).  With S = 1 there is no split-K
+// workspace and no merge.  (Each load of a tile must lie in one page:
+// block_size >= its rows.)  Returns S, or 0 for the stream-K plan.
+int segment_split(int kv_dtype, int head_size, int block_size, const HeadTiling &valu, int nseq,
+                  int num_kv_heads, long long max_ctx, int cus) {
+    const int tile = tile_tokens(head_size, kv_dtype, false);
+    const long long segs = (long long)nseq * num_kv_heads * valu.head_tiles;
+    if (valu.head_tile > xhip::kSegMaxHeadTile || block_size < tile / xhip::kLoadsPerTile ||
+        segs > cus)
+        return 0;
+    constexpr long long kSegSplitBytes = 160 << 10;
+    const long long cap = (long long)xhip::kSegWaves * xhip::kSegTiles * xhip::kSegRounds;
+    const long long seg_tiles = (max_ctx + tile - 1) / tile;
+    const long long seg_bytes = max_ctx * head_size * elem_bytes(kv_dtype) * 2;
+    int S = 1;
+    while (S < 4 && segs * S * 2 <= cus &&
+           (seg_bytes / (S * 2) >= kSegSplitBytes || seg_tiles > S * cap))
+        S *= 2;
+    return seg_tiles <= S * cap ? S : 0;
 }
 
 // Smallest stream-K range, in split units, the automatic plan gives a
@@ -284,6 +320,41 @@ constexpr long long kMaxLaunchTiles = 1LL << 30;  // bounds the partial workspac
 // such starts on one wavefront.  Explicit partition_tokens plans charge 0,
 // so each wavefront's range is exactly partition_tokens of K/V.
 constexpr int kSegmentCost = 2;
+
+// Whether an automatic plan of a use_mfma_auto shape takes the MFMA tiles.
+// Not where the batch takes the segment launch (whole outputs only), nor
+// where its 16-token tiles would pass the limit of split units that the VALU
+// tile's longer ones keep.  Else by group and by the K/V bytes the table
+// bounds.  The VALU tile waits for its loads before it computes, works per
+// query head, and reads K/V once per 8 of them; the MFMA tile costs the same
+// for up to 16 heads, with the next tile in flight, but its chain is longer,
+// so short batches of small groups stay.  Measured on MI355X (fp32, VALU ->
+// MFMA tiles, us a step):
+//   group 8, head_size 128: 1 x 96 tokens 13.2 -> 11.7, 8 sequences of
+//     300-900 tokens 25.6 -> 18.8; group 16, 32 of 64-2048: 69.6 -> 34.1;
+//   group 4: bounds of 15-30 MB 13.2 -> 14.2, 14.8 -> 15.8, 15.0 -> 15.7;
+//     59-65 MB 17.8 -> 17.0, 19.8 -> 18.3, 21.6 -> 20.3; 32 sequences of
+//     256-2048 tokens 64.4 -> 57.2;
+//   groups 1 and 2: 63-74 MB 14.4 -> 18.9, 16.8 -> 18.7; 109 MB 27.6 -> 27.1;
+//     218 MB 43.1 -> 38.9.
+bool auto_mfma(int kv_dtype, int head_size, int block_size, const HeadTiling &valu, int num_seqs,
+               int num_kv_heads, long long max_ctx, int cus, bool partial) {
+    if (!use_mfma_auto(kv_dtype, head_size, block_size)) return false;
+    if (!partial && segment_split(kv_dtype, head_size, block_size, valu, num_seqs, num_kv_heads,
+                                  max_ctx, cus) > 0)
+        return false;
+    const int heads = valu.head_tile * valu.head_tiles;  // the group, rounded up
+    if (heads <= 4) {
+        constexpr double kMinBytes = 32e6, kMinBytesNarrow = 128e6;
+        const double bytes = 2.0 * elem_bytes(kv_dtype) * head_size * num_kv_heads *
+                             (double)num_seqs * (double)max_ctx;
+        if (bytes < (heads <= 2 ? kMinBytesNarrow : kMinBytes)) return false;
+    }
+    HeadTiling t;
+    if (!head_tiling(heads, true, kv_dtype, head_size, &t)) return false;
+    const long long units = (max_ctx + 15) / 16 + kSegmentCost;
+    return (long long)num_kv_heads * t.head_tiles * units < kMaxLaunchTiles;
+}
 
 const char *dtype_name(int kv_dtype) {
     switch (kv_dtype) {
@@ -400,9 +471,9 @@ int run(void *out, const void *query, const void *key_cache, const void *value_c
     if (max_ctx > (1LL << 28))
         return set_status(NXT_ATTN_E_UNSUPPORTED, "context bound %lld tokens too large", max_ctx);
     const int group = num_heads / num_kv_heads;
-    const bool mfma = use_mfma(kv_dtype, head_size, block_size);
+    bool mfma = use_mfma(kv_dtype, head_size, block_size);
     HeadTiling tiling;
-    if (!head_tiling(group, mfma, head_size, &tiling))
+    if (!head_tiling(group, mfma, kv_dtype, head_size, &tiling))
         return set_status(NXT_ATTN_E_UNSUPPORTED, "GQA group %d > %d", group, max_group(mfma));
     if (nt && (num_seqs != 1 || !po || !out || rows || fold || partition_tokens ||
                !(head_size == 32 || head_size == 64 || head_size == 128) || !nt->k || !nt->v ||
@@ -425,7 +496,7 @@ int run(void *out, const void *query, const void *key_cache, const void *value_c
     if ((uintptr_t)block_tables & 3 || (uintptr_t)seq_lens & 3)
         return set_status(NXT_ATTN_E_INVALID, "int32 tables must be 4-byte aligned");
 
-    const int tile = tile_tokens(head_size, kv_dtype, mfma);
+    int tile = tile_tokens(head_size, kv_dtype, mfma);
     if (partition_tokens != 0 && (!is_pow2(partition_tokens) || partition_tokens < tile))
         return set_status(NXT_ATTN_E_UNSUPPORTED,
                           "partition_tokens %d must be a power of two >= %d for head_size %d %s",
@@ -436,6 +507,14 @@ int run(void *out, const void *query, const void *key_cache, const void *value_c
     if (e != hipSuccess) return set_status(NXT_ATTN_E_HIP, "hipGetDevice: %s", hipGetErrorString(e));
     hipStream_t stream = (hipStream_t)stream_handle;
     const int cus = cu_count(device);
+    // (explicit plans keep their tile)
+    if (partition_tokens == 0 &&
+        auto_mfma(kv_dtype, head_size, block_size, tiling, num_seqs, num_kv_heads, max_ctx, cus,
+                  po || fold)) {
+        mfma = true;
+        head_tiling(group, mfma, kv_dtype, head_size, &tiling);
+        tile = tile_tokens(head_size, kv_dtype, mfma);
+    }
     const int segs = num_kv_heads * tiling.head_tiles;
     const int seg_cost = partition_tokens == 0 ? kSegmentCost : 0;
     const long long units_per_seg = (max_ctx + tile - 1) / tile + seg_cost;
@@ -473,29 +552,12 @@ int run(void *out, const void *query, const void *key_cache, const void *value_c
                                   partition_tokens, waves);
         }
 
-        // Small batches on the VALU tile path: one round of workgroups over
-        // the segments (paged_decode_segment_kernel) when they fit one per
-        // CU, S of them per segment.  A workgroup streams its share of a
-        // segment through one CU (~68 GB/s measured on MI355X), so a segment
-        // is split while each share keeps at least kSegSplitBytes of K/V,
-        // which one CU streams in about the time the merge launch then
-        // needed takes (~2.3 us).  With S = 1 there is no split-K workspace
-        // and no merge.  (Each load of a tile must lie in one page:
-        // block_size >= its rows.)
-        long long seg_split = 0;  // 0: the stream-K plan
-        if (!mfma && partition_tokens == 0 && !po && !fold &&
-            tiling.head_tile <= xhip::kSegMaxHeadTile && block_size >= tile / xhip::kLoadsPerTile &&
-            (long long)nseq * segs <= cus) {
-            constexpr long long kSegSplitBytes = 160 << 10;
-            const long long cap = (long long)xhip::kSegWaves * xhip::kSegTiles * xhip::kSegRounds;
-            const long long seg_tiles = (max_ctx + tile - 1) / tile;
-            const long long seg_bytes = max_ctx * head_size * elem_bytes(kv_dtype) * 2;
-            long long S = 1;
-            while (S < 4 && (long long)nseq * segs * S * 2 <= cus &&
-                   (seg_bytes / (S * 2) >= kSegSplitBytes || seg_tiles > S * cap))
-                S *= 2;
-            if (seg_tiles <= S * cap) seg_split = S;
-        }
+        // (small batches on the VALU tile path: one round of workgroups)
+        const int seg_split =
+            !mfma && partition_tokens == 0 && !po && !fold
+                ? segment_split(kv_dtype, head_size, block_size, tiling, nseq, num_kv_heads,
+                                max_ctx, cus)
+                : 0;
         const bool seg_launch = seg_split > 0;
 
         const size_t eb_total = (size_t)elem_bytes(kv_dtype);
@@ -683,7 +745,7 @@ int cascade_run(void *out, const void *query, const void *key_cache, const void 
     long long fw = 0;
     bool inplan = false;  // the partition launch plans both batches itself
     if (wide && supported_head_size(head_size) &&
-        head_tiling(group, true, head_size, &stile)) {
+        head_tiling(group, true, kv_dtype, head_size, &stile)) {
         const long long tiles = ((long long)max_num_blocks_per_seq * block_size + 15) / 16 + kSegmentCost;
         const bool fits = v_max * (long long)num_kv_heads * (rows / 32) * tiles < kMaxLaunchTiles &&
                           (long long)num_seqs * num_kv_heads * stile.head_tiles * tiles <
@@ -1095,12 +1157,17 @@ __attribute__((visibility("default"))) int nxt_paged_attention_auto_waves(
         (kv_dtype != NXT_KV_FP16 && kv_dtype != NXT_KV_BF16 && kv_dtype != NXT_KV_FP32))
         return NXT_ATTN_E_INVALID;
     if (!is_pow2(block_size)) return NXT_ATTN_E_UNSUPPORTED;
-    const bool mfma = use_mfma(kv_dtype, head_size, block_size);
+    bool mfma = use_mfma(kv_dtype, head_size, block_size);
     HeadTiling tiling;
-    if (!head_tiling(num_heads / num_kv_heads, mfma, head_size, &tiling))
+    if (!head_tiling(num_heads / num_kv_heads, mfma, kv_dtype, head_size, &tiling))
         return NXT_ATTN_E_UNSUPPORTED;
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return NXT_ATTN_E_HIP;
+    if (auto_mfma(kv_dtype, head_size, block_size, tiling, num_seqs, num_kv_heads,
+                  (long long)max_num_blocks_per_seq * block_size, cu_count(device), false)) {
+        mfma = true;
+        head_tiling(num_heads / num_kv_heads, mfma, kv_dtype, head_size, &tiling);
+    }
     const int nseq = num_seqs < xhip::kMaxSeqsPerLaunch ? num_seqs : xhip::kMaxSeqsPerLaunch;
     const int tile = tile_tokens(head_size, kv_dtype, mfma);
     const long long ub = (long long)nseq * num_kv_heads * tiling.head_tiles *

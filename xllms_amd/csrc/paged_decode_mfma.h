@@ -1,5 +1,6 @@
-// MFMA tile path of the paged-decode attention (fp16 / bf16 K/V, head_size a
-// multiple of 32, block_size >= 16).  One wavefront serves R row blocks of 16
+// MFMA tile path of the paged-decode attention (head_size a multiple of 32,
+// block_size >= 16; fp16 / bf16 K/V, and fp32 up to head_size 128 in automatic
+// plans).  One wavefront serves R row blocks of 16
 // query heads of one kv head (R = 1, or 2 for groups of 17-32 heads at
 // head_size <= 128): every K/V tile it loads is used by all 16R heads.
 // Below, one row block; with R = 2 the QK^T MFMAs run once per block on the
@@ -31,6 +32,10 @@
 //         two-byte reads a lane to gather V^T) was 40 LDS instructions and a
 //         write-to-read wait in every tile's chain; fp16, head_size 128,
 //         16 x 1024 tokens, 32 / 8 heads: 21.3 -> 20.7 us a step.
+// fp32: v_mfma_f32_16x16x4 for both products, 16-byte chunks of 4 dims on
+// either side: QK^T step (c, i) multiplies element i of the K and Q chunks at
+// byte 64c + 16g, PV step r element e of the chunk of row 4g + r with P's row
+// 4g + r, so neither operand needs a permutation.
 // Loads are buffer loads: a token past the end of the range, or in a page
 // with a negative id, gets an out-of-range offset and reads as zero without
 // touching memory; its score is masked to -inf.  The next tile's K/V loads
@@ -101,6 +106,11 @@ template <int KV> __device__ __forceinline__ f32x4 mfma_pv(u32x2 a, u32x2 b, f32
                                                          __builtin_bit_cast(i16x4, b), c, 0, 0, 0);
 }
 
+// 16x16x4 (A lane: row j, k = g; B lane: column j, k = g).
+__device__ __forceinline__ f32x4 mfma_f32(uint32_t a, uint32_t b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a),
+                                                __builtin_bit_cast(float, b), c, 0, 0, 0);
+}
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const char *base) {
     return __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, 0x7FFFFFFF, 0x00020000);
@@ -292,12 +302,29 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
 
     // S = K Q^T for 16 tokens x 16 heads, per row block.
     f32x4 s[R];
+    if constexpr (KV == KV_F32) {
+        // four partial sums over the dims of a chunk's element: a chain of
+        // D/16 instead of D/4 dependent MFMAs, and as many fewer roundings
+        static_assert(R == 1, "fp32 tiles have one row block");
+        f32x4 part[4];
 #pragma unroll
-    for (int b = 0; b < R; b++) s[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < 4; i++) part[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int c = 0; c < G::kQkSteps; c++)
+        for (int c = 0; c < G::kQkSteps; c++) {
+            const u32x4 qc = q.get(qs, lane, 0, c);
 #pragma unroll
-        for (int b = 0; b < R; b++) s[b] = mfma_qk<KV>(r.k[c], q.get(qs, lane, b, c), s[b]);
+            for (int i = 0; i < 4; i++)
+                part[i] = mfma_f32(lane_word(r.k[c], i), lane_word(qc, i), part[i]);
+        }
+        s[0] = (part[0] + part[1]) + (part[2] + part[3]);
+    } else {
+#pragma unroll
+        for (int b = 0; b < R; b++) s[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int c = 0; c < G::kQkSteps; c++)
+#pragma unroll
+            for (int b = 0; b < R; b++) s[b] = mfma_qk<KV>(r.k[c], q.get(qs, lane, b, c), s[b]);
+    }
 
     bool ok[4];
 #pragma unroll
@@ -306,6 +333,7 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
     // Online softmax of head j over the four tokens of this lane; P in the
     // 16-bit type as hi + lo parts (B operand of the PV MFMA).
     u32x2 p_hi[R], p_lo[R];
+    float p32[4], alpha32 = 1.0f;  // fp32: P itself, and the rescale of the running output
 #pragma unroll
     for (int b = 0; b < R; b++) {
         float sc[4];
@@ -326,6 +354,12 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
         }
         st[b].l = st[b].l * alpha + psum;
         st[b].m = m_new;
+        if constexpr (KV == KV_F32) {
+            alpha32 = alpha;
+#pragma unroll
+            for (int i = 0; i < 4; i++) p32[i] = pe[i];
+            continue;
+        }
         // P = hi + lo in the 16-bit type (lo = the exact fp32 remainder of hi)
         const uint32_t h01 = pack16<KV>(pe[0], pe[1]), h23 = pack16<KV>(pe[2], pe[3]);
         const f32x2 r01 = unpack16<KV>(h01), r23 = unpack16<KV>(h23);
@@ -342,7 +376,9 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
     }
 
     // O^T += V^T P for every dim block: the block's dim of the lane's four
-    // token rows, a 16-bit half of one word of each row's chunk.
+    // token rows, a 16-bit half of one word of each row's chunk (fp32: a word
+    // of it; the tile's sum starts from zero and is then added to the rescaled
+    // running output, one rounding per tile in the long sum instead of 16).
     for_groups<KV, D>([&](auto vb) {
         constexpr int B = decltype(vb)::value;
         u32x4 v[4];
@@ -350,6 +386,15 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
         for (int i = 0; i < 4; i++) v[i] = vs.template chunk<B>(r, lane, i);
 #pragma unroll
         for (int e = 0; e < G::group_dims(B); e++) {
+            if constexpr (KV == KV_F32) {
+                f32x4 &o = st[0].o[G::kDims * B + e];
+                f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    t = mfma_f32(lane_word(v[i], e), __builtin_bit_cast(uint32_t, p32[i]), t);
+                o = o * alpha32 + t;
+                continue;
+            }
             const int n = G::kDims * B + e, w = e / 2;
             const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
             const u32x2 a = {__builtin_amdgcn_perm(lane_word(v[1], w), lane_word(v[0], w), sel),
@@ -572,7 +617,7 @@ __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPie
         // (the window is written and read by this wavefront: its LDS
         // accesses complete in order)
         __builtin_amdgcn_wave_barrier();
-        const size_t row_bytes = (size_t)D * 2;
+        const size_t row_bytes = MfmaGeometry<KV, D>::kRowBytes;
         const bool first = pc.kvh == 0 && pc.t_begin == 0;
 #pragma unroll
         for (int b = 0; b < R; b++) {
@@ -588,18 +633,19 @@ __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPie
             }
 #pragma unroll
             for (int c = 0; c < MfmaGeometry<KV, D>::kQkSteps; c++)
-                q[b][c] = src ? load16(src + (size_t)(32 * c + 8 * g) * 2) : u32x4{0, 0, 0, 0};
+                q[b][c] = src ? load16(src + 64 * c + 16 * g) : u32x4{0, 0, 0, 0};
         }
         return;
     }
     const int nh = min(kMfmaHeads * R, p.group - g0);
-    const char *q0 = q_row(p, pc.s, pc.kvh * p.group + g0, D, 2);
+    constexpr int RB = MfmaGeometry<KV, D>::kRowBytes;
+    const char *q0 = q_row(p, pc.s, pc.kvh * p.group + g0, D, MfmaGeometry<KV, D>::kElemBytes);
 #pragma unroll
     for (int b = 0; b < R; b++)
 #pragma unroll
         for (int c = 0; c < MfmaGeometry<KV, D>::kQkSteps; c++)
             q[b][c] = (16 * b + j < nh)
-                          ? load16(q0 + ((size_t)(16 * b + j) * D + 32 * c + 8 * g) * 2)
+                          ? load16(q0 + (size_t)(16 * b + j) * RB + 64 * c + 16 * g)
                           : u32x4{0, 0, 0, 0};
 }
 
@@ -924,7 +970,9 @@ __device__ __forceinline__ void mfma_partition_body(
     MfmaLds<KV, D, R, PAIR ? 0 : mfma_wg_fixup(kMfmaHeads * R, D)> &sm,
     const CascadeLdsPlan *cp = nullptr) {
     using G = MfmaGeometry<KV, D>;
+    constexpr int EB = G::kElemBytes;
     constexpr int FIX = PAIR ? 0 : mfma_wg_fixup(kMfmaHeads * R, D);
+    constexpr bool kFoldAhead = R == 1 && KV != KV_F32;  // (registers for it)
     constexpr int NW = kMfmaWavesPerGroup;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -987,8 +1035,8 @@ __device__ __forceinline__ void mfma_partition_body(
         int blk_a = __builtin_amdgcn_readlane(ids, 0);
         XHIP_WAVE_STAMP(p, wave, 0);
         {
-            const char *kb = (const char *)p.k + (size_t)pc.kvh * (size_t)p.kv_head_stride * 2;
-            const char *vb = (const char *)p.v + (size_t)pc.kvh * (size_t)p.kv_head_stride * 2;
+            const char *kb = (const char *)p.k + (size_t)pc.kvh * (size_t)p.kv_head_stride * EB;
+            const char *vb = (const char *)p.v + (size_t)pc.kvh * (size_t)p.kv_head_stride * EB;
             mfma_load_tile<KV, D>(p, kb, vb, pc.t_begin, pc.t_end, blk_a, lane, pc.s < p.cached_seqs,
                               ra);
         }
@@ -1003,10 +1051,10 @@ __device__ __forceinline__ void mfma_partition_body(
             const int ids_n = mfma_load_ids<SRC>(p, tables, pn, 0, lane, cp);
             const int fold_base_n =
                 (p.fold_row && has_next && pn.t_begin == 0) ? p.fold_row[pn.s] : -1;
-            const char *kb = (const char *)p.k + (size_t)pc.kvh * (size_t)p.kv_head_stride * 2;
-            const char *vb = (const char *)p.v + (size_t)pc.kvh * (size_t)p.kv_head_stride * 2;
-            const char *kb_n = (const char *)p.k + (size_t)pn.kvh * (size_t)p.kv_head_stride * 2;
-            const char *vb_n = (const char *)p.v + (size_t)pn.kvh * (size_t)p.kv_head_stride * 2;
+            const char *kb = (const char *)p.k + (size_t)pc.kvh * (size_t)p.kv_head_stride * EB;
+            const char *vb = (const char *)p.v + (size_t)pc.kvh * (size_t)p.kv_head_stride * EB;
+            const char *kb_n = (const char *)p.k + (size_t)pn.kvh * (size_t)p.kv_head_stride * EB;
+            const char *vb_n = (const char *)p.v + (size_t)pn.kvh * (size_t)p.kv_head_stride * EB;
             const bool cached = pc.s < p.cached_seqs;
             const bool cached_n = has_next && pn.s < p.cached_seqs;
             const int *bt = src_table<SRC>(p, tables, pc.s, cp);
@@ -1020,7 +1068,7 @@ __device__ __forceinline__ void mfma_partition_body(
             }
             MfmaFold<KV, D, R> fold;
             fold.base = fold_base;
-            if (R == 1 && fold.base >= 0) mfma_fold_load<KV, D, R>(p, pc, lane, fold);
+            if (kFoldAhead && fold.base >= 0) mfma_fold_load<KV, D, R>(p, pc, lane, fold);
             const int ntiles = (pc.t_end - pc.t_begin + 15) >> 4;
 #if XHIP_TRACING
             n_tiles += ntiles;
@@ -1048,7 +1096,7 @@ __device__ __forceinline__ void mfma_partition_body(
             }
 
             if (fold.base >= 0) {
-                if (R != 1) mfma_fold_load<KV, D, R>(p, pc, lane, fold);
+                if (!kFoldAhead) mfma_fold_load<KV, D, R>(p, pc, lane, fold);
                 mfma_fold_apply<KV, D, R>(fold, lane, st);
             }
             if (pc.whole) {
@@ -1177,10 +1225,19 @@ __device__ __forceinline__ void mfma_partition_body(
 }
 
 
-// Two wavefronts per SIMD (the plan's occupancy) up to head_size 128: at
-// most 256 registers each.  Larger heads need more and run one per SIMD.
+// Wavefronts per SIMD of the partition kernel, which the automatic plan
+// launches in one resident round: two where a tile is at most 8 KB, with at
+// most 256 registers each, else one.  Larger tiles need more registers, and
+// two wavefronts of two 16 KB tiles in flight each are more than HBM serves
+// evenly (fp32, head_size 128, 32 / 8 heads, 32 sequences of 256-2048 tokens:
+// the wavefronts' last tiles spread over 41-60 us, 67.5 us a step; one
+// wavefront per SIMD 46-52 us, 57.8 us a step).
+template <int KV, int D> constexpr int mfma_waves_per_simd() {
+    return MfmaGeometry<KV, D>::kRowBytes <= 256 ? 2 : 1;
+}
+
 template <int KV, int D, int R>
-__global__ __launch_bounds__(64 * kMfmaWavesPerGroup, D <= 128 ? 2 : 1) void paged_decode_partition_mfma_kernel(
+__global__ __launch_bounds__(64 * kMfmaWavesPerGroup, (mfma_waves_per_simd<KV, D>())) void paged_decode_partition_mfma_kernel(
     const DecodeParams p, const int *__restrict__ lens, const int *__restrict__ tables) {
     // lens / tables are p.seq_lens / p.block_tables again: as restrict
     // kernel arguments their wavefront-uniform reads become scalar loads,
