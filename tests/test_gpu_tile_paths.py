@@ -27,8 +27,8 @@ def _check(wl, what, **kw):
 
 
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
-@pytest.mark.parametrize("head_size", [32, 64, 96, 128, 192, 256])
-@pytest.mark.parametrize("group", [1, 4, 16, 20])
+@pytest.mark.parametrize("head_size", [32, 64, 80, 96, 112, 128, 192, 256])
+@pytest.mark.parametrize("group", [1, 3, 4, 16, 20])
 def test_tile_edges(cuda, dtype, head_size, group):
     lens = [1, 2, 3, 4, 5, 15, 16, 17, 31, 32, 33, 0, 255, 1025]
     for bs in (16, 32):

@@ -182,12 +182,14 @@ bool use_mfma(int kv_dtype, int head_size, int block_size) {
 }
 
 // Shapes outside use_mfma whose automatic stream-K plans may take the MFMA
-// tiles (auto_mfma): fp32 at head sizes whose tiles fit the registers.
-// Explicit partition_tokens plans keep the VALU tile, whose length is their
+// tiles (auto_mfma): fp32 at head sizes whose tiles fit the registers, and
+// fp16/bf16 at head sizes 80 and 112 (their V chunks padded).  Explicit partition_tokens plans keep the VALU tile, whose length is their
 // unit.
 bool use_mfma_auto(int kv_dtype, int head_size, int block_size) {
-    return kv_dtype == NXT_KV_FP32 && head_size % 32 == 0 &&
-           head_size <= xhip::kMfmaF32MaxHeadSize && block_size >= 16;
+    if (block_size < 16) return false;
+    return kv_dtype == NXT_KV_FP32
+               ? head_size % 32 == 0 && head_size <= xhip::kMfmaF32MaxHeadSize
+               : head_size == 80 || head_size == 112;
 }
 
 // Tokens per tile of the kernel instantiation: 16 on the MFMA path, else
@@ -217,7 +219,7 @@ bool head_tiling(int group, bool mfma, int kv_dtype, int head_size, HeadTiling *
         // K/V tile once for all of them (16-bit types, head_size <= 128),
         // else two wavefronts of one block each
         const bool wide = group > xhip::kMfmaHeads && kv_dtype != NXT_KV_FP32 &&
-                          head_size <= xhip::kMfmaWideMaxHeadSize;
+                          head_size % 32 == 0 && head_size <= xhip::kMfmaWideMaxHeadSize;
         t->head_tile = wide ? 2 * xhip::kMfmaHeads : xhip::kMfmaHeads;
         t->head_tiles = (group + t->head_tile - 1) / t->head_tile;
         return true;
@@ -275,10 +277,11 @@ int partition_occupancy(int kv_dtype, int head_size, int head_tile, bool mfma, s
     }
 }
 
-// Wavefronts per CU of the MFMA partition kernel's plan: eight (2 per SIMD).
-// Measured on MI355X against the twelve that fit: 4-10% less time on configs
-// 2, 3 and 4 (fewer concurrent page streams per HBM channel, and an even
-// finish across wavefronts).
+// Wavefronts per CU of the cascade's plans, and the most that the small-batch
+// bound of auto_waves is taken over: eight (2 per SIMD).  Measured on MI355X
+// against the twelve that fit: 4-10% less time on configs 2, 3 and 4 (fewer
+// concurrent page streams per HBM channel, and an even finish across
+// wavefronts).
 constexpr int kMfmaWavesPerCu = 8;
 
 int waves_per_group(bool mfma) { return mfma ? xhip::kMfmaWavesPerGroup : xhip::kWavesPerGroup; }
@@ -293,7 +296,10 @@ long long auto_waves(int kv_dtype, int head_size, int head_tile, bool mfma, int 
     if (occ <= 0) return 0;
     const int wpg = waves_per_group(mfma);
     int per_cu = occ * wpg;
-    if (mfma && per_cu > kMfmaWavesPerCu) per_cu = kMfmaWavesPerCu;
+    if (mfma) {
+        const int cap = 4 * xhip::mfma_waves_per_simd(head_size * elem_bytes(kv_dtype), head_tile);
+        if (per_cu > cap) per_cu = cap;
+    }
     long long w = (long long)cus * per_cu;
     // On the MFMA path a batch bounded below kSmallBatchUnits units per
     // wavefront of that round gets one workgroup per CU instead: its wavefronts are short
@@ -303,7 +309,8 @@ long long auto_waves(int kv_dtype, int head_size, int head_tile, bool mfma, int 
     // 16.9 us, 2 x 8192 22.5 -> 21.6 us; 1 x 2048 and batches above the bound
     // unchanged.
     constexpr long long kSmallBatchUnits = 8;
-    if (mfma && ub_tiles < kSmallBatchUnits * w && per_cu > wpg) w = (long long)cus * wpg;
+    const long long w_small = (long long)cus * (per_cu < kMfmaWavesPerCu ? per_cu : kMfmaWavesPerCu);
+    if (mfma && ub_tiles < kSmallBatchUnits * w_small && per_cu > wpg) w = (long long)cus * wpg;
     const long long need = (ub_tiles + kMinTilesPerWave - 1) / kMinTilesPerWave;
     if (need < w) w = need;
     w = (w + wpg - 1) / wpg * wpg;
@@ -337,6 +344,11 @@ constexpr int kSegmentCost = 2;
 //     256-2048 tokens 64.4 -> 57.2;
 //   groups 1 and 2: 63-74 MB 14.4 -> 18.9, 16.8 -> 18.7; 109 MB 27.6 -> 27.1;
 //     218 MB 43.1 -> 38.9.
+// fp16/bf16 at head sizes 80 and 112, from groups of 3: group 3, head_size
+// 112, 24 sequences of 100-2000 tokens 30.5 -> 28.1, 30 of 10-60 13.1 -> 12.5;
+// group 8, head_size 80, 1 x 96 tokens 15.2 -> 11.9, 4 of 300-900 17.2 -> 11.9;
+// group 20, 16 of 300-2000 29.9 -> 14.8.  Groups 1 and 2 stay on the VALU
+// tiles: 32 / 32 heads, head_size 80, 24 of 100-2000 49.9 against 55.1.
 bool auto_mfma(int kv_dtype, int head_size, int block_size, const HeadTiling &valu, int num_seqs,
                int num_kv_heads, long long max_ctx, int cus, bool partial) {
     if (!use_mfma_auto(kv_dtype, head_size, block_size)) return false;
@@ -344,7 +356,9 @@ bool auto_mfma(int kv_dtype, int head_size, int block_size, const HeadTiling &va
                                   max_ctx, cus) > 0)
         return false;
     const int heads = valu.head_tile * valu.head_tiles;  // the group, rounded up
-    if (heads <= 4) {
+    if (kv_dtype != NXT_KV_FP32) {
+        if (heads <= 2) return false;
+    } else if (heads <= 4) {
         constexpr double kMinBytes = 32e6, kMinBytesNarrow = 128e6;
         const double bytes = 2.0 * elem_bytes(kv_dtype) * head_size * num_kv_heads *
                              (double)num_seqs * (double)max_ctx;

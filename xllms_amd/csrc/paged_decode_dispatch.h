@@ -23,13 +23,13 @@ static const void *valu_fn(int head_tile) {
 }
 
 template <int KV, int D> constexpr bool has_mfma() {
-    return D % 32 == 0 && (KV != KV_F32 || D <= kMfmaF32MaxHeadSize);
+    return KV == KV_F32 ? D % 32 == 0 && D <= kMfmaF32MaxHeadSize : D % 16 == 0;
 }
 
 // Two row blocks per wavefront (head tile 32) fit the register file at two
 // wavefronts per SIMD for the 16-bit types up to head_size 128.
 template <int KV, int D> constexpr bool has_mfma_wide() {
-    return KV != KV_F32 && has_mfma<KV, D>() && D <= kMfmaWideMaxHeadSize;
+    return KV != KV_F32 && D % 32 == 0 && D <= kMfmaWideMaxHeadSize;
 }
 
 template <int KV, int D>

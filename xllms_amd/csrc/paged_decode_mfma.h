@@ -1,6 +1,6 @@
-// MFMA tile path of the paged-decode attention (head_size a multiple of 32,
-// block_size >= 16; fp16 / bf16 K/V, and fp32 up to head_size 128 in automatic
-// plans).  One wavefront serves R row blocks of 16
+// MFMA tile path of the paged-decode attention (block_size >= 16; fp16 / bf16
+// K/V at head sizes that are multiples of 32, and in automatic plans at 80 and
+// 112 and fp32 up to head_size 128).  One wavefront serves R row blocks of 16
 // query heads of one kv head (R = 1, or 2 for groups of 17-32 heads at
 // head_size <= 128): every K/V tile it loads is used by all 16R heads.
 // Below, one row block; with R = 2 the QK^T MFMAs run once per block on the
@@ -64,12 +64,16 @@ template <int KV, int D> struct MfmaGeometry {
     static constexpr int kQkSteps = (kRowBytes + 63) / 64;  // 16-byte K loads per lane
     // V rows: groups of 16 chunks, a lane holding one chunk of each group (of
     // its four token rows); full groups have kDims dims (16 bytes) per chunk,
-    // the last one as many as the row still has.
+    // the last one as many as the row still has.  An odd count of 16-bit dims
+    // (head sizes 80, 112) is padded: whole chunks, of which the last lanes'
+    // lie past the row (kPadded; their rows of the blocks are never used).
     static constexpr int kDims = 16 / kElemBytes;
     static constexpr int kVGroups = (D + 16 * kDims - 1) / (16 * kDims);
     static constexpr int group_dims(int b) {
-        return (D - 16 * kDims * b) / 16 < kDims ? (D - 16 * kDims * b) / 16 : kDims;
+        const int r = (D - 16 * kDims * b) / 16;
+        return r >= kDims || (kElemBytes == 2 && r % 2) ? kDims : r;
     }
+    static constexpr bool kPadded = kElemBytes == 2 && (D / 16) % 2 != 0;
     static constexpr int group_words(int b) { return group_dims(b) * kElemBytes / 4; }
     static constexpr int kDimBlocks = kDims * (kVGroups - 1) + group_dims(kVGroups - 1);
     // Rows of fewer than 16 chunks of 16 bytes: the tile is loaded in whole
@@ -77,8 +81,8 @@ template <int KV, int D> struct MfmaGeometry {
     // loads, one per token row, are slower: head_size 32, bf16, 64 sequences
     // of 256-4096 tokens, 32 / 8 heads 39.4 us a step).
     static constexpr bool kVStaged = kRowBytes < 256;
-    static constexpr int kVLoads = kVStaged ? kRowBytes / 64 : 4 * kVGroups;
-    static_assert(D % 32 == 0, "MFMA path needs head_size % 32 == 0");
+    static constexpr int kVLoads = kVStaged ? (kRowBytes + 63) / 64 : 4 * kVGroups;
+    static_assert(D % 16 == 0 && (!kPadded || kVStaged), "head sizes of the MFMA path");
 };
 
 // First of the group_dims(b) dims of chunk i of V group b: element e of the
@@ -173,12 +177,14 @@ __device__ __forceinline__ void mfma_issue_loads(__amdgpu_buffer_rsrc_t rk,
     const bool krow_ok = kt < n;
 #pragma unroll
     for (int c = 0; c < G::kQkSteps; c++)
-        r.k[c] = buf_load<4, POLICY>(rk, krow_ok ? (uint32_t)(kt * RB + 64 * c + 16 * g) : kOobOffset);
+        r.k[c] = buf_load<4, POLICY>(rk, krow_ok && (RB % 64 == 0 || 64 * c + 16 * g < RB)
+                                             ? (uint32_t)(kt * RB + 64 * c + 16 * g)
+                                             : kOobOffset);
     if constexpr (G::kVStaged) {
 #pragma unroll
         for (int c = 0; c < G::kVLoads; c++) {
             const int at = 1024 * c + 16 * lane;
-            r.v[c] = buf_load<4, POLICY>(rv, at / RB < n ? (uint32_t)at : kOobOffset);
+            r.v[c] = buf_load<4, POLICY>(rv, at < min(n, G::kTile) * RB ? (uint32_t)at : kOobOffset);
         }
     } else {
         for_groups<KV, D>([&](auto b) {
@@ -254,7 +260,9 @@ template <int KV, int D> struct MfmaVLds<KV, D, true> {
         const uint32_t *src = (const uint32_t *)t +
                               tile_token(lane >> 4, i) * (G::kRowBytes / 4) + W * (lane & 15);
         u32x4 x;
-        if constexpr (W == 2) {
+        if constexpr (W == 4) {
+            x = *(const u32x4 *)src;
+        } else if constexpr (W == 2) {
             const u32x2 y = *(const u32x2 *)src;
             x = __builtin_shufflevector(y, y, 0, 1, -1, -1);
         } else {
@@ -595,6 +603,10 @@ __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPie
                                             const CascadeLdsPlan *cp = nullptr) {
     const int j = lane & 15, g = lane >> 4;
     const int g0 = pc.ht * kMfmaHeads * R;
+    auto q_chunk_ok = [](int c, int gr) {
+        constexpr int RBQ = MfmaGeometry<KV, D>::kRowBytes;
+        return RBQ % 64 == 0 || 64 * c + 16 * gr < RBQ;
+    };
     if constexpr (SRC == kSrcPrefix) {
         const int *d = cp->vdesc + 4 * pc.s;
         const int vbase = __builtin_amdgcn_readfirstlane(d[0]);
@@ -633,7 +645,7 @@ __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPie
             }
 #pragma unroll
             for (int c = 0; c < MfmaGeometry<KV, D>::kQkSteps; c++)
-                q[b][c] = src ? load16(src + 64 * c + 16 * g) : u32x4{0, 0, 0, 0};
+                q[b][c] = src && q_chunk_ok(c, g) ? load16(src + 64 * c + 16 * g) : u32x4{0, 0, 0, 0};
         }
         return;
     }
@@ -644,7 +656,7 @@ __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPie
     for (int b = 0; b < R; b++)
 #pragma unroll
         for (int c = 0; c < MfmaGeometry<KV, D>::kQkSteps; c++)
-            q[b][c] = (16 * b + j < nh)
+            q[b][c] = (16 * b + j < nh && q_chunk_ok(c, g))
                           ? load16(q0 + (size_t)(16 * b + j) * RB + 64 * c + 16 * g)
                           : u32x4{0, 0, 0, 0};
 }
@@ -677,8 +689,9 @@ __device__ __forceinline__ void mfma_fold_load(const DecodeParams &p, const Mfma
             constexpr int B = decltype(vb)::value, N = G::group_dims(B);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                float x[N];
-                load_floats(p.fold_out + r * D + mfma_dim<KV, D>(B, 4 * g + i), x);
+                const int d = mfma_dim<KV, D>(B, 4 * g + i);
+                float x[N] = {};
+                if (!G::kPadded || d < D) load_floats(p.fold_out + r * D + d, x);
 #pragma unroll
                 for (int e = 0; e < N; e++) f.o[b][G::kDims * B + e][i] = x[e];
             }
@@ -747,6 +760,7 @@ __device__ __forceinline__ void mfma_write_rows(const DecodeParams &p, const Mfm
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int d = mfma_dim<KV, D>(B, 4 * gq + i);
+                if (G::kPadded && d >= D) continue;
                 float f[N];
                 state_dims<KV, D, B>(st[b], i, f);
 #pragma unroll
@@ -785,6 +799,7 @@ __device__ __forceinline__ void mfma_write_partial(const DecodeParams &p, const 
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int d = mfma_dim<KV, D>(B, 4 * gq + i);
+                if (G::kPadded && d >= D) continue;
                 float f[N];
                 state_dims<KV, D, B>(st[b], i, f);
                 if constexpr (HS) {
@@ -895,7 +910,9 @@ __device__ __forceinline__ void absorb_partial(const DecodeParams &p, int slot, 
             constexpr int B = decltype(vb)::value, N = G::group_dims(B);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const size_t at = row + mfma_dim<KV, D>(B, 4 * gq + i);
+                const int d = mfma_dim<KV, D>(B, 4 * gq + i);
+                if (G::kPadded && d >= D) continue;
+                const size_t at = row + d;
                 float x[N];
                 if constexpr (HS) {
 #pragma unroll
@@ -1225,19 +1242,8 @@ __device__ __forceinline__ void mfma_partition_body(
 }
 
 
-// Wavefronts per SIMD of the partition kernel, which the automatic plan
-// launches in one resident round: two where a tile is at most 8 KB, with at
-// most 256 registers each, else one.  Larger tiles need more registers, and
-// two wavefronts of two 16 KB tiles in flight each are more than HBM serves
-// evenly (fp32, head_size 128, 32 / 8 heads, 32 sequences of 256-2048 tokens:
-// the wavefronts' last tiles spread over 41-60 us, 67.5 us a step; one
-// wavefront per SIMD 46-52 us, 57.8 us a step).
-template <int KV, int D> constexpr int mfma_waves_per_simd() {
-    return MfmaGeometry<KV, D>::kRowBytes <= 256 ? 2 : 1;
-}
-
 template <int KV, int D, int R>
-__global__ __launch_bounds__(64 * kMfmaWavesPerGroup, (mfma_waves_per_simd<KV, D>())) void paged_decode_partition_mfma_kernel(
+__global__ __launch_bounds__(64 * kMfmaWavesPerGroup, (mfma_waves_per_simd(MfmaGeometry<KV, D>::kRowBytes, kMfmaHeads * R))) void paged_decode_partition_mfma_kernel(
     const DecodeParams p, const int *__restrict__ lens, const int *__restrict__ tables) {
     // lens / tables are p.seq_lens / p.block_tables again: as restrict
     // kernel arguments their wavefront-uniform reads become scalar loads,
