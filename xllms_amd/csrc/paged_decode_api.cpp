@@ -811,7 +811,7 @@ int cascade_run(void *out, const void *query, const void *key_cache, const void 
                  o_xp = fw ? take(4 * ((size_t)v_max + 2)) : 0,
                  o_yo = fw ? take(4 * 2 * (size_t)fw * gts * head_size) : 0,
                  o_ym = fw ? take(4 * 2 * (size_t)fw * gts * 2) : 0,
-                 o_yp = fw ? take(4 * ((size_t)num_seqs + 1)) : 0,
+                 o_yp = fw ? take(4 * ((size_t)num_seqs + 2)) : 0,
                  o_so = fw ? take(4 * (size_t)num_seqs * num_heads * head_size) : 0,
                  o_sl2 = fw ? take(4 * (size_t)num_seqs * num_heads) : 0;
     // held over the plan and both passes (they read what the plan wrote)

@@ -88,11 +88,24 @@ template <int KV, int D, int RS> union MfmaLdsPair {
     MfmaLds<KV, D, RS> b;
 };
 
+// The units per range of both batches, for the merge (in place of its own
+// divisions: its code comes from a cold cache, and at 3.9 KB instead of 6.2 a
+// step over 256 sequences in 16 groups, fp16, takes 108.3 us instead of
+// 109.5), stored after the workgroup's ranges.  tp / ts: the batches' units; gp of G workgroups are the prefix's.
+__device__ __forceinline__ void cascade_publish_ranges(const DecodeParams &pp,
+                                                       const DecodeParams &ps, int tp, int ts,
+                                                       int gp, int G) {
+    constexpr int NW = kMfmaWavesPerGroup;
+    if (gp > 0)
+        pp.ws_prefix[pp.num_seqs + 1] = tiles_per_wave(tp, gp * NW >> 1, pp.min_tiles_per_wave);
+    if (G > gp)
+        ps.ws_prefix[ps.num_seqs + 1] = tiles_per_wave(ts, (G - gp) * NW, ps.min_tiles_per_wave);
+}
+
 // Partition launch over both batches.  pp / ps are the prefix and suffix
 // batches' plans; their num_waves is the whole launch's (gridDim.x *
-// kMfmaWavesPerGroup).  Workgroup 0 also stores both unit prefixes and the
-// prefix body's workgroup count (pp.ws_prefix[pp.num_seqs + 1]) for the
-// merge.
+// kMfmaWavesPerGroup).  Workgroup 0 also stores both unit prefixes and, after
+// them, each batch's units per range for the merge.
 template <int KV, int D, int RS>
 __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, 2) void paged_decode_cascade_mfma_kernel(
     const DecodeParams pp, const DecodeParams ps, const int *__restrict__ plens,
@@ -107,7 +120,6 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, 2) void paged_decode_casca
     const int G = gridDim.x;
     const int gp = cascade_prefix_groups(pre_p[pp.num_seqs], pre_s[ps.num_seqs], G,
                                          ps.min_tiles_per_wave);
-    if (blockIdx.x == 0 && threadIdx.x == 0) pp.ws_prefix[pp.num_seqs + 1] = gp;
     // neighbouring logical workgroups share an XCD (and its L2).  (Giving
     // every XCD its share of prefix workgroups instead measured 0.5-1 us
     // slower.)
@@ -118,6 +130,8 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, 2) void paged_decode_casca
     else
         mfma_partition_body<KV, D, RS, false, kSrcBatch, KV == KV_F16>(
             ps, slens, stables, pre_s, l - gp, (G - gp) * NW, sm.b);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        cascade_publish_ranges(pp, ps, pre_p[pp.num_seqs], pre_s[ps.num_seqs], gp, G);
 }
 
 // In-kernel plan.  With at most kInPlanGroupsMax groups, every workgroup of
@@ -137,8 +151,8 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, 2) void paged_decode_casca
 // members its query rows belong to when it starts (mfma_load_q, kSrcPrefix):
 // the members of a group are ranked in sequence order, so the rows a piece
 // computes are the same members' in every workgroup.  Workgroup 0 also
-// stores what the merge reads: both unit prefixes, the split and the
-// batches' lengths; p_row, every member's first row in the prefix batch, is
+// stores what the merge reads: both unit prefixes, the units per range and
+// the batches' lengths; p_row, every member's first row in the prefix batch, is
 // stored by the piece that starts its prefix-batch sequence (kv head 0), and
 // -1 for every other sequence by workgroup 0.
 // LDS ints of the in-kernel plan: B caller sequences, V prefix-batch
@@ -281,7 +295,6 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, 2) void paged_decode_casca
     if (blockIdx.x == 0) {
         for (int v = tid; v <= V; v += NT) pp.ws_prefix[v] = pre_p[v];
         for (int q = tid; q <= B; q += NT) ps.ws_prefix[q] = pre_s[q];
-        if (tid == 0) pp.ws_prefix[V + 1] = gp;
         for (int v = tid; v < V; v += NT) const_cast<int *>(pp.seq_lens)[v] = vlen[v];
         for (int q = tid; q < B; q += NT) {
             const_cast<int *>(ps.seq_lens)[q] = slen[q];
@@ -298,6 +311,8 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, 2) void paged_decode_casca
     else
         mfma_partition_body<KV, D, RS, false, kSrcSuffix, KV == KV_F16>(
             ps, nullptr, tables, pre_s, l - gp, (Gw - gp) * NW, sm.b, &cp);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        cascade_publish_ranges(pp, ps, pre_p[pp.num_seqs], pre_s[ps.num_seqs], gp, Gw);
     XHIP_WG_FLUSH(pp);
 }
 
@@ -312,6 +327,10 @@ __device__ __forceinline__ void absorb_row(float lse, const f32x4 &row, float &m
     m = M;
 }
 
+// Query rows per kv head of a prefix-batch sequence of the fused launch: two
+// 32-row head tiles.
+constexpr int kCascadeFusedRows = 4 * kMfmaHeads;
+
 // The state of one float4 column of a segment of batch p: its partials when
 // the partition left the segment cut, else its finished row.  seg is the
 // segment's index within its sequence, hrow the column's head in the
@@ -320,7 +339,7 @@ __device__ __forceinline__ void absorb_row(float lse, const f32x4 &row, float &m
 // head tile pair_ht.  HS: the states are fp16 (DecodeParams::out_h, ws_h).
 template <int GT, int D, bool HS>
 __device__ __forceinline__ void segment_state(const DecodeParams &p, int s, int L, int seg,
-                                              int pre_s, int total, int waves, size_t row, int hrow,
+                                              int pre_s, int tpw, size_t row, int hrow,
                                               int c, float &m, float &l, f32x4 &acc,
                                               int pair_ht = -1) {
     const int Ts = (L + 15) / 16;
@@ -328,14 +347,11 @@ __device__ __forceinline__ void segment_state(const DecodeParams &p, int s, int 
     PartialSlots ps;
     const bool cut =
         pair_ht >= 0
-            ? segment_partials_paired(seg_start, seg_start + p.seg_cost, Ts,
-                                      tiles_per_wave(total, waves >> 1, p.min_tiles_per_wave),
-                                      pair_ht, ps)
-            : segment_partials<kMfmaWavesPerGroup>(
-                  p, seg_start, seg_start + p.seg_cost, Ts,
-                  tiles_per_wave(total, waves, p.min_tiles_per_wave), ps);
+            ? segment_partials_paired(seg_start, seg_start + p.seg_cost, Ts, tpw, pair_ht, ps)
+            : segment_partials<kMfmaWavesPerGroup>(p, seg_start, seg_start + p.seg_cost, Ts, tpw,
+                                                   ps);
     if (cut) {
-        merge_partials<GT, D, 8, HS>(p, ps, 0, 1, hrow * 2, hrow * D + c * 4, m, l, acc);
+        merge_partials<GT, D, 4, HS>(p, ps, 0, 1, hrow * 2, hrow * D + c * 4, m, l, acc);
     } else {
         const float lse = p.out_lse[row];
         const f32x4 o = HS ? unpack_h4(*(const u32x2 *)((const char *)p.out_h + (row * D + c * 4) * 2))
@@ -348,14 +364,13 @@ __device__ __forceinline__ void segment_state(const DecodeParams &p, int s, int 
 // heads), NT threads striding over its float4 columns, writing the output
 // rows of ps (ps.out or ps.o_rows; its partial-output buffers hold the
 // suffix states).  p_row[s] is the row,
-// in the prefix batch's rows of a kv head laid end to end (`rows` per
-// prefix-batch sequence), of s's first query head; -1: s has no prefix.
+// in the prefix batch's rows of a kv head laid end to end (kCascadeFusedRows
+// per prefix-batch sequence), of s's first query head; -1: s has no prefix.
 template <int KV, int D, int GTS, int NT>
 __global__ __launch_bounds__(NT) void paged_decode_cascade_merge_kernel(
-    const DecodeParams pp, const DecodeParams ps, const int *__restrict__ p_row, int rows) {
+    const DecodeParams pp, const DecodeParams ps, const int *__restrict__ p_row) {
     XHIP_MERGE_SCOPE(pp);
     constexpr int C4 = D / 4;
-    constexpr int NW = kMfmaWavesPerGroup;
     constexpr int GTP = 2 * kMfmaHeads;
     constexpr bool HS = KV == KV_F16;  // fp16 states (set by the host for fp16 K/V)
     // The prefix batch's lengths and unit prefixes, loaded with the first
@@ -369,46 +384,43 @@ __global__ __launch_bounds__(NT) void paged_decode_cascade_merge_kernel(
             l_vpre[v] = pp.ws_prefix[v];
         }
     }
-    const int segs = ps.num_kv_heads * ps.head_tiles;
-    const int s = blockIdx.x / segs;
-    const int seg = blockIdx.x - s * segs;
-    const int kvh = seg / ps.head_tiles;
-    const int g0 = (seg - kvh * ps.head_tiles) * GTS;
-    const int nh = min(GTS, ps.group - g0);
-    const int ncols = nh * C4;
+    const int s = blockIdx.y, seg = blockIdx.x;
     // the scalars, requested together
     const int Ls = seq_len_of(ps, s);
     const int fb = p_row[s];
-    const int tot_s = ps.ws_prefix[ps.num_seqs];
     const int pre_s = ps.ws_prefix[s];
-    const int tot_p = pp.ws_prefix[pp.num_seqs];
-    const int gp = pp.ws_prefix[pp.num_seqs + 1];
-    asm volatile("" ::"s"(Ls), "s"(fb), "s"(tot_s), "s"(pre_s), "s"(tot_p), "s"(gp));
+    const int tpw_s = ps.ws_prefix[ps.num_seqs + 1];
+    const int tpw_p = pp.ws_prefix[pp.num_seqs + 1];
+    asm volatile("" ::"s"(Ls), "s"(fb), "s"(pre_s), "s"(tpw_s), "s"(tpw_p));
+    int kvh = seg, g0 = 0;
+    if (ps.head_tiles != 1) {
+        kvh = seg / ps.head_tiles;
+        g0 = (seg - kvh * ps.head_tiles) * GTS;
+    }
+    const int nh = min(GTS, ps.group - g0);
+    const int ncols = nh * C4;
     __syncthreads();
-    const int G = ps.num_waves / NW;
     const size_t srow0 = (size_t)s * ps.num_heads + (size_t)kvh * ps.group + g0;
     for (int col = threadIdx.x; col < ncols; col += NT) {
         const int h = col / C4, c = col - h * C4;
         float m = -INFINITY, l = 0.0f;
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
         if (Ls > 0)
-            segment_state<GTS, D, HS>(ps, s, Ls, seg, pre_s, tot_s, (G - gp) * NW, srow0 + h, h,
-                                      c, m, l, acc);
+            segment_state<GTS, D, HS>(ps, s, Ls, seg, pre_s, tpw_s, srow0 + h, h, c, m, l, acc);
         if (fb >= 0) {
-            const int q = fb + g0 + h;
-            const int v = q / rows, j = q - v * rows;
+            const uint32_t q = (uint32_t)(fb + g0 + h);
+            const int v = (int)(q / kCascadeFusedRows), j = (int)(q % kCascadeFusedRows);
             const int Lv = v_lds ? l_vlen[v] : seq_len_of(pp, v);
             if (Lv > 0) {
                 const int htp = j / GTP;
-                const size_t prow = (size_t)v * pp.num_heads + (size_t)kvh * rows + j;
+                const size_t prow =
+                    (size_t)v * pp.num_heads + (size_t)kvh * kCascadeFusedRows + j;
                 segment_state<GTP, D, HS>(pp, v, Lv, kvh, v_lds ? l_vpre[v] : pp.ws_prefix[v],
-                                          tot_p, gp * NW, prow, j - htp * GTP, c, m, l, acc, htp);
+                                          tpw_p, prow, j - htp * GTP, c, m, l, acc, htp);
             }
         }
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        char *orow = o_row(ps, s, kvh * ps.group + g0 + h, D, 2);
-#pragma unroll
-        for (int e = 0; e < 4; e++) store_elem<KV>(orow, c * 4 + e, acc[e] * inv);
+        store4<KV>(o_row(ps, s, kvh * ps.group + g0 + h, D, 2), c * 4,
+                   acc * (l > 0.0f ? 1.0f / l : 0.0f));
     }
 }
 
@@ -416,6 +428,7 @@ template <int KV, int D, int RS>
 static hipError_t launch_cascade_attn_rs(const DecodeParams &pp, const DecodeParams &ps,
                                          const int *p_row, int rows, const CascadeInPlan *ip,
                                          hipStream_t st, hipEvent_t ev_start, hipEvent_t ev_stop) {
+    if (rows != kCascadeFusedRows) return hipErrorInvalidValue;
     const unsigned grid = (unsigned)(ps.num_waves / kMfmaWavesPerGroup);
     const dim3 block(64 * kMfmaWavesPerGroup);
     // the merge reads fp16 states exactly when the K/V are fp16
@@ -448,9 +461,9 @@ static hipError_t launch_cascade_attn_rs(const DecodeParams &pp, const DecodePar
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const unsigned segs = (unsigned)(ps.num_seqs * ps.num_kv_heads * ps.head_tiles);
+    const dim3 segs((unsigned)(ps.num_kv_heads * ps.head_tiles), (unsigned)ps.num_seqs);
     paged_decode_cascade_merge_kernel<KV, D, kMfmaHeads * RS, 128>
-        <<<segs, 128, 0, st>>>(pp, ps, p_row, rows);
+        <<<segs, 128, 0, st>>>(pp, ps, p_row);
     return hipGetLastError();
 }
 

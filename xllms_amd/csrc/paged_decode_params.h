@@ -49,8 +49,7 @@ constexpr int kSegTiles = 2;
 constexpr int kSegRounds = 4;
 constexpr int kSegMaxHeadTile = 2;
 
-// Workgroup-level combine of cut segments (MFMA tile path, head_size <=
-// 128): the kMfmaWavesPerGroup wavefronts of a workgroup own consecutive
+// Workgroup-level combine of cut segments (MFMA tile path): the kMfmaWavesPerGroup wavefronts of a workgroup own consecutive
 // stream-K ranges, so the pieces of one segment that fall in one workgroup
 // are merged through LDS at the end of the kernel.  Only one fp32 partial
 // per (segment, workgroup it spans) is left for the merge kernel, in the
@@ -58,9 +57,12 @@ constexpr int kSegMaxHeadTile = 2;
 // inside one workgroup is written finished.  Mode 1 (one row block): every
 // wavefront has an LDS slot.  Mode 2 (two row blocks, whose slots would
 // not leave room for two workgroups per CU): one relay slot per workgroup.
-// 0: no combine (head_size > 128).
+// 0: no combine (head_size 256: its 66 KB of slots cost more than the partials
+// of small groups; bf16, 16 / 8 heads, 24 sequences of 77-3001 tokens 33.8 us
+// a step with it, 32.5 without; head_size 192, 48 / 8 heads, 32 of 100-3000
+// 56.1 with, 56.9 without).
 constexpr int mfma_wg_fixup(int rows_per_tile, int head_size) {
-    return head_size > 128 ? 0 : rows_per_tile == kMfmaHeads ? 1 : 2;
+    return head_size > 192 ? 0 : rows_per_tile == kMfmaHeads ? 1 : 2;
 }
 
 // Wavefronts per SIMD of the MFMA partition kernel, which the automatic plan
