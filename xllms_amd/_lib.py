@@ -21,6 +21,7 @@ BACKEND_TRACE_SO = os.path.join(LIB_DIR, "libxllm_hip_backend_trace.so")
 
 _lock = threading.Lock()
 _cache: dict[str, ctypes.CDLL] = {}
+_product: ctypes.CDLL | None = None  # the typed product library
 
 c_int = ctypes.c_int
 c_void_p = ctypes.c_void_p
@@ -96,6 +97,9 @@ _LEGACY_ARGS = [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
 def backend(trace: bool = False) -> ctypes.CDLL:
     """The product library, or with trace=True its instrumented build (the
     same entry points plus xhip_set_wg_trace / xhip_wg_trace_words)."""
+    global _product
+    if _product is not None and not trace:
+        return _product  # loaded and typed: every operator call comes through here
     lib = _load(BACKEND_TRACE_SO if trace else BACKEND_SO)
     if trace and not getattr(lib, "_xllm_trace_typed", False):
         lib.xhip_set_wg_trace.argtypes = [c_void_p]
@@ -145,6 +149,8 @@ def backend(trace: bool = False) -> ctypes.CDLL:
         lib.nxt_activation_ex.restype = c_int
         _type_kv_index(lib)
         lib._xllm_typed = True
+    if not trace:
+        _product = lib
     return lib
 
 

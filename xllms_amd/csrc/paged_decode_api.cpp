@@ -547,9 +547,19 @@ int run(void *out, const void *query, const void *key_cache, const void *value_c
     for (int s0 = 0; s0 < num_seqs; s0 += per_launch) {
         const int nseq = num_seqs - s0 < per_launch ? num_seqs - s0 : per_launch;
         const long long ub_tiles = (long long)nseq * seq_units;
+        // (small batches on the VALU tile path: one round of workgroups)
+        const int seg_split =
+            !mfma && partition_tokens == 0 && !po && !fold
+                ? segment_split(kv_dtype, head_size, block_size, tiling, nseq, num_kv_heads,
+                                max_ctx, cus)
+                : 0;
+        const bool seg_launch = seg_split > 0;
         long long waves;
         int min_tpw;
-        if (partition_tokens == 0) {
+        if (seg_launch) {  // (its grid is the segments': no wavefront count to plan)
+            waves = 0;
+            min_tpw = kMinTilesPerWave;
+        } else if (partition_tokens == 0) {
             waves = auto_waves(kv_dtype, head_size, tiling.head_tile, mfma, nseq, ub_tiles, cus);
             if (waves <= 0)
                 return set_status(NXT_ATTN_E_HIP, "no occupancy for head_size %d %s", head_size,
@@ -565,14 +575,6 @@ int run(void *out, const void *query, const void *key_cache, const void *value_c
                                   "partition_tokens %d gives %lld wavefronts; raise it",
                                   partition_tokens, waves);
         }
-
-        // (small batches on the VALU tile path: one round of workgroups)
-        const int seg_split =
-            !mfma && partition_tokens == 0 && !po && !fold
-                ? segment_split(kv_dtype, head_size, block_size, tiling, nseq, num_kv_heads,
-                                max_ctx, cus)
-                : 0;
-        const bool seg_launch = seg_split > 0;
 
         const size_t eb_total = (size_t)elem_bytes(kv_dtype);
         // workspace: fp32 partials o, their (m, l), the unit prefix; under a

@@ -41,10 +41,15 @@ class PagedAttentionError(RuntimeError):
         self.status = status
 
 
+_dtype_codes: dict = {}  # torch dtype -> code, filled on first use (torch is imported lazily)
+
+
 def kv_dtype_of(tensor) -> int:
-    import torch
-    return {torch.float16: NXT_KV_FP16, torch.bfloat16: NXT_KV_BF16,
-            torch.float32: NXT_KV_FP32}[tensor.dtype]
+    if not _dtype_codes:
+        import torch
+        _dtype_codes.update({torch.float16: NXT_KV_FP16, torch.bfloat16: NXT_KV_BF16,
+                             torch.float32: NXT_KV_FP32})
+    return _dtype_codes[tensor.dtype]
 
 
 def last_status() -> tuple[int, str]:
@@ -61,8 +66,12 @@ def _ptr(t) -> int:
 
 
 def _stream_handle(stream) -> int:
-    import torch
     if stream is None:
+        # the current stream's handle without building a Stream object around
+        # it (the operators' host time is what bounds their smallest calls)
+        import torch
+        if torch.cuda.is_initialized():
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
         stream = torch.cuda.current_stream()
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
