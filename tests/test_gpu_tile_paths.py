@@ -66,3 +66,33 @@ def test_fp32_tile_path_rule(cuda, case):
     wl = W.small_case(num_seqs=n, H=H, KVH=KVH, D=128, kv_dtype=W.FP32, seed=n + tokens, lens=lens)
     print(f"case H={H} KVH={KVH} seqs={n} tokens={tokens}", flush=True)
     _check(wl, f"H={H} KVH={KVH} seqs={n} tokens={tokens}")
+
+
+@pytest.mark.parametrize("n", [2, 31, 33, 130, 1025])
+def test_detection_run_lengths(cuda, n):
+    """Shared runs one page either side of the 16 pages the detection compares
+    at a time, up to the whole table, over batches around its hash table's
+    sizes; lengths that end inside a run."""
+    import numpy as np
+    import torch
+
+    from tests.cascade_cases import detect_prefix_groups
+    rng = np.random.default_rng(n)
+    width, bs = 50, 16
+    tables = rng.permutation(n * width).reshape(n, width).astype(np.int32)
+    runs = [1, 15, 16, 17, 31, 32, 33, 49, 50]
+    for s in range(1, n):
+        if s % 5 != 4:  # shares the first pages of a leader a few rows up
+            lead = s - s % 5
+            k = runs[s % len(runs)]
+            if lead != s:
+                tables[s, :k] = tables[lead, :k]
+    lens = rng.integers(1, width * bs + 1, size=n).astype(np.int32)
+    lens[: min(n, 30)] = width * bs
+    group, blocks, count = PA.prefix_groups(torch.from_numpy(tables).cuda(),
+                                            torch.from_numpy(lens).cuda(), block_size=bs)
+    torch.cuda.synchronize()
+    want_group, want_blocks = detect_prefix_groups(tables, lens, bs)
+    assert int(count[0]) == len(want_blocks)
+    assert np.array_equal(group.cpu().numpy(), want_group)
+    assert np.array_equal(blocks.cpu().numpy()[: len(want_blocks)], want_blocks)
