@@ -96,3 +96,29 @@ def test_detection_run_lengths(cuda, n):
     assert int(count[0]) == len(want_blocks)
     assert np.array_equal(group.cpu().numpy(), want_group)
     assert np.array_equal(blocks.cpu().numpy()[: len(want_blocks)], want_blocks)
+
+
+@pytest.mark.parametrize("key,scale", [(4e36, 4.0), (3e38, 1.0), (-3e38, 1.0)])
+def test_fp32_overflowing_scores(cuda, key, scale):
+    """A score that overflows when scaled, or already as a sum (to +inf: NaN
+    rows; to -inf: a weight of zero): the matrix tiles (automatic plan) against
+    the VALU tiles (explicit plan), NaN for NaN."""
+    import torch
+    wl = W.small_case(num_seqs=2, H=16, KVH=2, D=64, kv_dtype=W.FP32, seed=7, lens=[40, 33])
+    dw = W.upload(wl)
+    dw.query.fill_(1.0)
+    dw.key_cache.mul_(0.01)
+    page = int(dw.block_tables[0, 1])
+    dw.key_cache[page, 0, 3] = key  # token 19 of sequence 0, kv head 0
+
+    def run(**kw):
+        dw.out.zero_()
+        PA.paged_attention(dw.out, dw.query, dw.key_cache, dw.value_cache, dw.block_tables,
+                           dw.seq_lens, num_kv_heads=2, scale=scale, **kw)
+        torch.cuda.synchronize()
+        return dw.out.clone().view(2, 16, 64)
+    auto, valu = run(), run(partition_tokens=256)
+    print(f"case key={key} scale={scale}", flush=True)
+    assert bool(torch.isnan(auto[0, :8]).all()) == (key > 0)
+    assert torch.equal(torch.isnan(auto), torch.isnan(valu))
+    assert torch.allclose(auto.nan_to_num(), valu.nan_to_num(), rtol=1e-5, atol=1e-6)

@@ -311,20 +311,29 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
     // S = K Q^T for 16 tokens x 16 heads, per row block.
     f32x4 s[R];
     if constexpr (KV == KV_F32) {
-        // four partial sums over the dims of a chunk's element: a chain of
-        // D/16 instead of D/4 dependent MFMAs, and as many fewer roundings
+        // A sum per chunk and element of a chunk (four products), added up as a
+        // tree: chains of D / 16 MFMAs carried more rounding into the scores
+        // than the VALU tile's sums over lanes do (error against 64 bits,
+        // 64 / 8 heads, head_size 128: VALU 2.2e-7, sums of two chunks 1.9e-7,
+        // of one 1.8e-7 with the exponent below).  The matrix cores wait for HBM
+        // here: the adds cost little (the 32-sequence batch of 256-2048 tokens,
+        // 32 / 8 heads: 56.9-57.4 us a step before, 57.3-58.0 after; VALU 63.4).
         static_assert(R == 1, "fp32 tiles have one row block");
-        f32x4 part[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) part[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        f32x4 part[G::kQkSteps];
 #pragma unroll
         for (int c = 0; c < G::kQkSteps; c++) {
             const u32x4 qc = q.get(qs, lane, 0, c);
+            f32x4 x[4];
 #pragma unroll
             for (int i = 0; i < 4; i++)
-                part[i] = mfma_f32(lane_word(r.k[c], i), lane_word(qc, i), part[i]);
+                x[i] = mfma_f32(lane_word(r.k[c], i), lane_word(qc, i), f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+            part[c] = (x[0] + x[1]) + (x[2] + x[3]);
         }
-        s[0] = (part[0] + part[1]) + (part[2] + part[3]);
+#pragma unroll
+        for (int w = 1; w < G::kQkSteps; w <<= 1)
+#pragma unroll
+            for (int c = 0; c + w < G::kQkSteps; c += 2 * w) part[c] += part[c + w];
+        s[0] = part[0];
     } else {
 #pragma unroll
         for (int b = 0; b < R; b++) s[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -357,7 +366,12 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
         float psum = 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            pe[i] = fast_exp2(sc[i] - ms);
+            float x = sc[i] - ms;
+            // fp32: the scaled score's own rounding stays out of the exponent
+            // (an infinite maximum keeps the difference, which is then NaN)
+            if constexpr (KV == KV_F32)
+                x = ok[i] && ms < INFINITY ? fmaf(s[b][i], p.scale_log2, -ms) : x;
+            pe[i] = fast_exp2(x);
             psum += pe[i];
         }
         st[b].l = st[b].l * alpha + psum;
