@@ -183,8 +183,8 @@ bool use_mfma(int kv_dtype, int head_size, int block_size) {
 
 // Shapes outside use_mfma whose automatic stream-K plans may take the MFMA
 // tiles (auto_mfma): fp32 at head sizes whose tiles fit the registers, and
-// fp16/bf16 at head sizes 80 and 112 (their V chunks padded).  Explicit partition_tokens plans keep the VALU tile, whose length is their
-// unit.
+// fp16/bf16 at head sizes 80 and 112 (their V chunks padded).  Explicit
+// partition_tokens plans keep the VALU tile, whose length is their unit.
 bool use_mfma_auto(int kv_dtype, int head_size, int block_size) {
     if (block_size < 16) return false;
     return kv_dtype == NXT_KV_FP32
