@@ -238,6 +238,14 @@ template <int KV, int D, int R> struct MfmaQLds<KV, D, R, true> {
     u32x4 q[R][MfmaGeometry<KV, D>::kQkSteps][64];
 };
 
+// Between LDS accesses of different lanes of one wavefront.  The wavefront's
+// LDS accesses complete in order, so there is nothing to wait for; but the
+// compiler orders two accesses only where one lane's addresses may meet, and
+// a word that another lane wrote never does.  (No instruction at this scope.)
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+}
+
 // The V tile of a wavefront where it is staged (MfmaGeometry::kVStaged), row-major.
 template <int KV, int D, bool STAGED = MfmaGeometry<KV, D>::kVStaged> struct MfmaVLds {
     __device__ __forceinline__ void put(const MfmaTileRegs<KV, D> &, int) {}
@@ -250,8 +258,10 @@ template <int KV, int D, bool STAGED = MfmaGeometry<KV, D>::kVStaged> struct Mfm
 template <int KV, int D> struct MfmaVLds<KV, D, true> {
     u32x4 t[64 * MfmaGeometry<KV, D>::kVLoads];
     __device__ __forceinline__ void put(const MfmaTileRegs<KV, D> &r, int lane) {
+        wave_lds_fence();  // after the last tile's chunks
 #pragma unroll
         for (int c = 0; c < MfmaGeometry<KV, D>::kVLoads; c++) t[64 * c + lane] = r.v[c];
+        wave_lds_fence();  // before this tile's
     }
     template <int B>
     __device__ __forceinline__ u32x4 chunk(const MfmaTileRegs<KV, D> &, int lane, int i) const {
@@ -631,6 +641,7 @@ __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPie
         const int r_lo = row0 / G, r_hi = min((row0 + 16 * R - 1) / G, count - 1);
         int *win = cp->win + (threadIdx.x >> 6) * (16 * R);
         int acc = 0;
+        wave_lds_fence();  // after the last piece's lookups
         for (int c0 = 0; c0 < cp->num_seqs && acc <= r_hi; c0 += 64) {
             const int s = c0 + lane;
             const bool in = s < cp->num_seqs && cp->grp[s] == gid;
@@ -640,8 +651,7 @@ __device__ __forceinline__ void mfma_load_q(const DecodeParams &p, const MfmaPie
             if (in && rk >= r_lo && rk <= r_hi) win[rk - r_lo] = s;
             acc += __popcll(m);
         }
-        // (the window is written and read by this wavefront: its LDS
-        // accesses complete in order)
+        wave_lds_fence();
         __builtin_amdgcn_wave_barrier();
         const size_t row_bytes = MfmaGeometry<KV, D>::kRowBytes;
         const bool first = pc.kvh == 0 && pc.t_begin == 0;
