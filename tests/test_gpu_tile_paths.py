@@ -122,3 +122,34 @@ def test_fp32_overflowing_scores(cuda, key, scale):
     assert bool(torch.isnan(auto[0, :8]).all()) == (key > 0)
     assert torch.equal(torch.isnan(auto), torch.isnan(valu))
     assert torch.allclose(auto.nan_to_num(), valu.nan_to_num(), rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("size", [1e5, 1e7, 1e9, 1e12, 1e16, 1e30])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_fp32_large_scores(cuda, size, sign):
+    """Finite scores so large that the rounding of a scaled score is far above
+    1 (log2 units): the largest score of a row still has a weight of 1 and the
+    others one of at most 1, as in the VALU tiles (explicit plan), where the
+    weights come from the differences of the rounded scores.  The scores are
+    size times 1, 1.5 or 2 times a head's factor, exact in fp32 before the
+    scale, so every weight is 0 or 1 and both paths average the same rows:
+    fp32 sums of at most 40 terms, 40 * 2^-24 < 1e-5."""
+    import torch
+    wl = W.small_case(num_seqs=2, H=16, KVH=2, D=64, kv_dtype=W.FP32, seed=11, lens=[40, 33])
+    dw = W.upload(wl)
+    dw.query.zero_()
+    dw.query.view(2, 16, 64)[:, :, 5] = torch.arange(1, 17, device="cuda") * float(size) * sign
+    tokens = torch.arange(dw.key_cache.shape[0] * 16, device="cuda").view(-1, 1, 16) * 7 % 3
+    dw.key_cache.zero_()
+    dw.key_cache[:, :, :, 5] = 1.0 + 0.5 * tokens
+
+    def run(**kw):
+        dw.out.zero_()
+        PA.paged_attention(dw.out, dw.query, dw.key_cache, dw.value_cache, dw.block_tables,
+                           dw.seq_lens, num_kv_heads=2, scale=0.125, **kw)
+        torch.cuda.synchronize()
+        return dw.out.clone()
+    auto, valu = run(), run(partition_tokens=256)
+    print(f"case size={size} sign={sign}", flush=True)
+    assert bool(torch.isfinite(valu).all()) and bool(torch.isfinite(auto).all())
+    assert torch.allclose(auto, valu, rtol=1e-5, atol=1e-5)

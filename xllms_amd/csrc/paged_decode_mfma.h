@@ -377,10 +377,13 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             float x = sc[i] - ms;
-            // fp32: the scaled score's own rounding stays out of the exponent
-            // (an infinite maximum keeps the difference, which is then NaN)
+            // fp32: the scaled score's own rounding stays out of the exponent.
+            // From 2^23 on half a unit of the maximum's last place is no
+            // longer small (at 2^33 it is 2^9: a weight of exp2(512), or of 0
+            // for the largest score), and the difference of the rounded
+            // scores, at most 0, is kept; so is an infinite maximum's (NaN).
             if constexpr (KV == KV_F32)
-                x = ok[i] && ms < INFINITY ? fmaf(s[b][i], p.scale_log2, -ms) : x;
+                x = ok[i] && fabsf(ms) < 8388608.0f ? fmaf(s[b][i], p.scale_log2, -ms) : x;
             pe[i] = fast_exp2(x);
             psum += pe[i];
         }
