@@ -153,3 +153,83 @@ def test_fp32_large_scores(cuda, size, sign):
     print(f"case size={size} sign={sign}", flush=True)
     assert bool(torch.isfinite(valu).all()) and bool(torch.isfinite(auto).all())
     assert torch.allclose(auto, valu, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("head_size", [80, 112])
+def test_weights_kept_in_fp32(cuda, dtype, head_size):
+    """The weights of automatic plans at head sizes 80 and 112 are fp32 on
+    either tile path: the values of three tokens cancel to about 2^-17 (bf16)
+    or 2^-20 (fp16) of their size, so a weight of 16 bits shows in the output.
+    Against 64 bits: a weight's relative error is below 2^-21 (the roundings
+    of the scale, of two scaled scores of up to 3 and of exp2, each 2^-24),
+    applied to the three weighted values, and the output's own rounding."""
+    import numpy as np
+    import torch
+    n, L, group, scale = 16, 40, 8, 0.75
+    wl = W.small_case(num_seqs=n, H=2 * group, KVH=2, D=head_size, kv_dtype=DT[dtype], seed=3,
+                      lens=[L] * n)
+    dw = W.upload(wl)
+    torch_dt = dw.query.dtype
+
+    def rnd(x):
+        return torch.from_numpy(x).to(torch_dt).double().numpy()
+    rng = np.random.default_rng(head_size)
+    dw.query.zero_()
+    dw.query.view(n, 2 * group, head_size)[:, ::group, 0] = 1.0  # the first head of a kv head
+    score = rnd(rng.uniform(-2.0, 0.0, (n, L)))
+    a, b, c = 1, 18, 37  # in three tiles, the largest score last
+    for t, lo in ((a, -1.5), (b, -0.5), (c, 1.0)):
+        score[:, t] = rnd(rng.uniform(lo, lo + 0.5, n))
+    w = np.exp(scale * (score - score[:, c:c + 1]))
+    v = np.zeros((n, L, head_size))
+    v[:, a] = rnd(rng.uniform(0.5, 1.0, (n, head_size)))
+    v[:, b] = -rnd(v[:, a] * (w[:, a] / w[:, b])[:, None])
+    v[:, c] = -rnd(v[:, a] * w[:, a, None] + v[:, b] * w[:, b, None])
+    K = np.zeros((n, L, head_size))
+    K[:, :, 0] = score
+    for cache, rows in ((dw.key_cache, K), (dw.value_cache, v)):
+        rows = torch.from_numpy(rows).to(torch_dt).cuda()
+        for t in range(L):
+            cache[dw.block_tables[:, t // 16].long(), :, t % 16] = rows[:, None, t]
+    want = np.einsum("nt,ntd->nd", w, v) / w.sum(1)[:, None]
+    size = np.einsum("nt,ntd->nd", w, np.abs(v)) / w.sum(1)[:, None]
+    bound = size * 2.0 ** -21 + np.abs(want) * 2.0 ** (-8 if dtype == "bf16" else -11) + \
+        (2.0 ** -25 if dtype == "fp16" else 0.0)  # (fp16: the smallest outputs' spacing)
+    for part in (0, 256):
+        dw.out.zero_()
+        PA.paged_attention(dw.out, dw.query, dw.key_cache, dw.value_cache, dw.block_tables,
+                           dw.seq_lens, num_kv_heads=2, scale=scale, partition_tokens=part)
+        torch.cuda.synchronize()
+        got = dw.out.view(n, 2 * group, head_size)[:, ::group].double().cpu().numpy()
+        worst = float((np.abs(got - want[:, None]) / bound[:, None]).max())
+        print(f"case {dtype} d={head_size} partition={part}: {worst:.3f} of the bound", flush=True)
+        assert worst <= 1.0
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("head_size", [80, 112])
+def test_infinite_values(cuda, dtype, head_size):
+    """An infinite value under a weight above 0 makes its output element
+    infinite, under the automatic plan as in the VALU tiles (explicit plan):
+    no part of a weight is 0."""
+    import torch
+    wl = W.small_case(num_seqs=2, H=16, KVH=2, D=head_size, kv_dtype=DT[dtype], seed=5,
+                      lens=[40, 33])
+    dw = W.upload(wl)
+    page = int(dw.block_tables[0, 1])
+    dw.value_cache[page, 0, 3, 7] = float("inf")      # token 19 of sequence 0, kv head 0
+    dw.value_cache[page, 1, 5, 70] = float("-inf")    # token 21, kv head 1
+
+    def run(**kw):
+        dw.out.zero_()
+        PA.paged_attention(dw.out, dw.query, dw.key_cache, dw.value_cache, dw.block_tables,
+                           dw.seq_lens, num_kv_heads=2, scale=0.01, **kw)
+        torch.cuda.synchronize()
+        return dw.out.clone().view(2, 16, head_size)
+    auto, valu = run(), run(partition_tokens=256)
+    print(f"case {dtype} d={head_size}", flush=True)
+    assert bool((auto[0, :8, 7] == float("inf")).all())
+    assert bool((auto[0, 8:, 70] == float("-inf")).all())
+    assert int(torch.isfinite(auto).logical_not().sum()) == 16
+    assert torch.equal(torch.isfinite(auto), torch.isfinite(valu))

@@ -344,11 +344,14 @@ constexpr int kSegmentCost = 2;
 //     256-2048 tokens 64.4 -> 57.2;
 //   groups 1 and 2: 63-74 MB 14.4 -> 18.9, 16.8 -> 18.7; 109 MB 27.6 -> 27.1;
 //     218 MB 43.1 -> 38.9.
-// fp16/bf16 at head sizes 80 and 112, from groups of 3: group 3, head_size
-// 112, 24 sequences of 100-2000 tokens 30.5 -> 28.1, 30 of 10-60 13.1 -> 12.5;
-// group 8, head_size 80, 1 x 96 tokens 15.2 -> 11.9, 4 of 300-900 17.2 -> 11.9;
-// group 20, 16 of 300-2000 29.9 -> 14.8.  Groups 1 and 2 stay on the VALU
-// tiles: 32 / 32 heads, head_size 80, 24 of 100-2000 49.9 against 55.1.
+// fp16/bf16, with the weights in fp32 as on the VALU tiles (32 fp32 MFMAs a
+// tile: beside HBM they count from ~40 us on).  Head_size 80 from groups of 3
+// (24 / 8 and 32 / 8 heads, 1-128 sequences, tables of 4 MB to 1 GB filled by
+// a 16th to all: 0.78-1.04 of the VALU tiles' time, 0.94 on average; 32 of
+// 1552 tokens 30.6 -> 27.4 us); 32 / 32 heads, groups of 1, 49.9 against 55.1.
+// Head_size 112 from groups of 5 (0.53-0.84: 32 of 1104 tokens, 40 / 8 heads,
+// 42.7 -> 28.5); groups of 3 and 4 lose up to 15% once HBM is busy (the same
+// with 24 / 8 heads 26.7 -> 28.9, 32 of 4464 63.9 -> 73.0) and gain 5% below.
 bool auto_mfma(int kv_dtype, int head_size, int block_size, const HeadTiling &valu, int num_seqs,
                int num_kv_heads, long long max_ctx, int cus, bool partial) {
     if (!use_mfma_auto(kv_dtype, head_size, block_size)) return false;
@@ -357,7 +360,7 @@ bool auto_mfma(int kv_dtype, int head_size, int block_size, const HeadTiling &va
         return false;
     const int heads = valu.head_tile * valu.head_tiles;  // the group, rounded up
     if (kv_dtype != NXT_KV_FP32) {
-        if (heads <= 2) return false;
+        if (heads <= (head_size == 80 ? 2 : 4)) return false;
     } else if (heads <= 4) {
         constexpr double kMinBytes = 32e6, kMinBytesNarrow = 128e6;
         const double bytes = 2.0 * elem_bytes(kv_dtype) * head_size * num_kv_heads *

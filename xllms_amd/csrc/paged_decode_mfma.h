@@ -17,7 +17,8 @@
 //         j+48 (4 each): in-lane max, two xor shuffles, exp2, running sum.
 //   PV    O^T[dim][head] += sum_t V[t][dim] P[head][t]
 //         v_mfma_f32_16x16x16 per dim block (twice: P = P_hi + P_lo in the
-//         16-bit type, so the product keeps ~22 bits of P): B = P, which is
+//         16-bit type, so the product keeps ~22 bits of P over fp16 and ~16
+//         over bf16, of a result with 11 and 8): B = P, which is
 //         exactly the C layout of the QK^T step (lane: head j, rows
 //         4g..4g+3); A = V^T (lane: one dim per block, the same four tokens).
 //         Which dim a lane holds in which block is free, so lane (g, j) loads
@@ -36,6 +37,8 @@
 // either side: QK^T step (c, i) multiplies element i of the K and Q chunks at
 // byte 64c + 16g, PV step r element e of the chunk of row 4g + r with P's row
 // 4g + r, so neither operand needs a permutation.
+// fp16 / bf16 at head sizes 80 and 112 (kP32): PV as for fp32, on V's elements
+// converted as they leave the chunk.
 // Loads are buffer loads: a token past the end of the range, or in a page
 // with a negative id, gets an out-of-range offset and reads as zero without
 // touching memory; its score is masked to -inf.  The next tile's K/V loads
@@ -74,6 +77,11 @@ template <int KV, int D> struct MfmaGeometry {
         return r >= kDims || (kElemBytes == 2 && r % 2) ? kDims : r;
     }
     static constexpr bool kPadded = kElemBytes == 2 && (D / 16) % 2 != 0;
+    // P in fp32 (v_mfma_f32_16x16x4 for PV): fp32 K/V, and the 16-bit head
+    // sizes whose explicit plans run the VALU tiles (80, 112), where P is fp32
+    // too: two 16-bit parts are ~22 bits of P for fp16, 16 for bf16, and a V
+    // of infinity times a part that is 0 is NaN.
+    static constexpr bool kP32 = KV == KV_F32 || kPadded;
     static constexpr int group_words(int b) { return group_dims(b) * kElemBytes / 4; }
     static constexpr int kDimBlocks = kDims * (kVGroups - 1) + group_dims(kVGroups - 1);
     // Rows of fewer than 16 chunks of 16 bytes: the tile is loaded in whole
@@ -114,6 +122,16 @@ template <int KV> __device__ __forceinline__ f32x4 mfma_pv(u32x2 a, u32x2 b, f32
 __device__ __forceinline__ f32x4 mfma_f32(uint32_t a, uint32_t b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a),
                                                 __builtin_bit_cast(float, b), c, 0, 0, 0);
+}
+
+// Element e of a chunk, in fp32.
+template <int KV> __device__ __forceinline__ uint32_t chunk_elem(u32x4 v, int e) {
+    if constexpr (KV == KV_F32) {
+        return lane_word(v, e);
+    } else {
+        const f32x2 x = unpack16<KV>(lane_word(v, e / 2));
+        return __builtin_bit_cast(uint32_t, e & 1 ? x.y : x.x);
+    }
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const char *base) {
@@ -360,7 +378,7 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
     // Online softmax of head j over the four tokens of this lane; P in the
     // 16-bit type as hi + lo parts (B operand of the PV MFMA).
     u32x2 p_hi[R], p_lo[R];
-    float p32[4], alpha32 = 1.0f;  // fp32: P itself, and the rescale of the running output
+    float p32[4], alpha32 = 1.0f;  // kP32: P itself, and the rescale of the running output
 #pragma unroll
     for (int b = 0; b < R; b++) {
         float sc[4];
@@ -389,7 +407,8 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
         }
         st[b].l = st[b].l * alpha + psum;
         st[b].m = m_new;
-        if constexpr (KV == KV_F32) {
+        if constexpr (G::kP32) {
+            static_assert(R == 1, "fp32 P: one row block");
             alpha32 = alpha;
 #pragma unroll
             for (int i = 0; i < 4; i++) p32[i] = pe[i];
@@ -411,9 +430,10 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
     }
 
     // O^T += V^T P for every dim block: the block's dim of the lane's four
-    // token rows, a 16-bit half of one word of each row's chunk (fp32: a word
-    // of it; the tile's sum starts from zero and is then added to the rescaled
-    // running output, one rounding per tile in the long sum instead of 16).
+    // token rows, a 16-bit half of one word of each row's chunk.  kP32: the
+    // element in fp32, one 16x16x4 per row; the tile's sum starts from zero
+    // and is then added to the rescaled running output, one rounding per tile
+    // in the long sum instead of 16.
     for_groups<KV, D>([&](auto vb) {
         constexpr int B = decltype(vb)::value;
         u32x4 v[4];
@@ -421,12 +441,12 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
         for (int i = 0; i < 4; i++) v[i] = vs.template chunk<B>(r, lane, i);
 #pragma unroll
         for (int e = 0; e < G::group_dims(B); e++) {
-            if constexpr (KV == KV_F32) {
+            if constexpr (G::kP32) {
                 f32x4 &o = st[0].o[G::kDims * B + e];
                 f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int i = 0; i < 4; i++)
-                    t = mfma_f32(lane_word(v[i], e), __builtin_bit_cast(uint32_t, p32[i]), t);
+                    t = mfma_f32(chunk_elem<KV>(v[i], e), __builtin_bit_cast(uint32_t, p32[i]), t);
                 o = o * alpha32 + t;
                 continue;
             }
