@@ -17,11 +17,17 @@ pytestmark = pytest.mark.gpu
 DT = {"fp16": W.FP16, "bf16": W.BF16, "fp32": W.FP32}
 
 
-def _check(wl, what, **kw):
+def _check(wl, what, tokens=0, **kw):
+    """Against the oracle; tokens: under a table that bounds at least so many
+    (the fp32 rule goes by the table)."""
     import torch
     dw = W.upload(wl)
-    PA.paged_attention(dw.out, dw.query, dw.key_cache, dw.value_cache, dw.block_tables,
-                       dw.seq_lens, num_kv_heads=wl.num_kv_heads, scale=wl.scale, **kw)
+    n, used = dw.block_tables.shape
+    bs = dw.key_cache.shape[2]
+    tables = torch.full((n, max(used, -(-tokens // bs))), -1, dtype=torch.int32, device="cuda")
+    tables[:, :used] = dw.block_tables
+    PA.paged_attention(dw.out, dw.query, dw.key_cache, dw.value_cache, tables, dw.seq_lens,
+                       num_kv_heads=wl.num_kv_heads, scale=wl.scale, **kw)
     torch.cuda.synchronize()
     assert_close(dw.out.float().cpu().numpy(), O.run_workload(wl, precision="mt"), wl.kv_dtype, what)
 
@@ -41,31 +47,47 @@ def test_tile_edges(cuda, dtype, head_size, group):
 @pytest.mark.parametrize("head_size", [32, 64, 96, 128])
 @pytest.mark.parametrize("group", [5, 8, 16, 17, 32])
 def test_fp32_tile_edges(cuda, head_size, group):
-    """fp32 automatic plans take the matrix tiles for groups above 4 at any
-    length: edges of the 16-token tile, one and two head tiles, pages of one
-    and two tiles."""
+    """fp32 automatic plans take the matrix tiles for groups above 4 (at head
+    sizes of more than 64 where the table bounds 64 MB): edges of the 16-token
+    tile, one and two head tiles, pages of one and two tiles."""
     lens = [1, 2, 3, 4, 5, 15, 16, 17, 31, 32, 33, 0, 255, 1025]
     for bs in (16, 32):
         wl = W.small_case(num_seqs=len(lens), H=2 * group, KVH=2, D=head_size, bs=bs,
                           kv_dtype=W.FP32, seed=head_size + group + bs, lens=lens)
         print(f"case fp32 d={head_size} group={group} bs={bs}", flush=True)
-        _check(wl, f"fp32 d={head_size} group={group} bs={bs}")
+        _check(wl, f"fp32 d={head_size} group={group} bs={bs}", tokens=4096)
 
 
 @pytest.mark.parametrize("case", [
-    # (H, KVH, seqs, tokens): fp32, head_size 128, batches just below and
-    # above the K/V bytes from which groups of up to 4 (32 MB) and up to 2
-    # (128 MB) take the matrix tiles; 33 kv heads x 8 sequences are more
-    # segments than CUs (no segment launch)
-    (8, 2, 15, 1024), (8, 2, 16, 1024), (33, 33, 8, 464), (33, 33, 8, 480), (34, 17, 16, 448),
-    (34, 17, 16, 480),
+    # (H, KVH, head_size, sequences, tokens the table bounds, matrix tiles?):
+    # either side of the fp32 rule's lines.  Groups of 3 and 4: 512 MB of K/V
+    # and 512 tokens at head sizes of more than 64, else 256 MB.  Groups from
+    # 5: 64 MB there, 16 MB for at most 112 tokens.  Groups of 1 and 2: never.
+    (32, 8, 128, 32, 1952, False), (32, 8, 128, 32, 1968, True),
+    (32, 8, 128, 128, 496, False), (32, 8, 128, 128, 512, True),
+    (12, 4, 128, 64, 1952, False), (12, 4, 128, 64, 1968, True),
+    (32, 8, 96, 32, 2592, False), (32, 8, 96, 32, 2608, True),
+    (16, 4, 64, 64, 1952, False), (16, 4, 64, 64, 1968, True),
+    (64, 8, 128, 8, 976, False), (64, 8, 128, 8, 992, True),
+    (64, 8, 128, 16, 112, False), (64, 8, 128, 32, 64, True), (64, 8, 128, 32, 128, False),
+    (64, 4, 128, 16, 976, False), (64, 4, 128, 16, 992, True),
+    (16, 8, 128, 64, 4096, False), (32, 32, 128, 64, 4096, False), (12, 12, 64, 64, 8192, False),
 ])
 def test_fp32_tile_path_rule(cuda, case):
-    H, KVH, n, tokens = case
-    lens = [max(1, tokens - 67 * i) for i in range(n)]
-    wl = W.small_case(num_seqs=n, H=H, KVH=KVH, D=128, kv_dtype=W.FP32, seed=n + tokens, lens=lens)
-    print(f"case H={H} KVH={KVH} seqs={n} tokens={tokens}", flush=True)
-    _check(wl, f"H={H} KVH={KVH} seqs={n} tokens={tokens}")
+    """The tile path on either side of each line, by the number of wavefronts
+    of its plan, and the outputs of a batch that fills little of such a
+    table."""
+    import torch
+    H, KVH, D, n, ctx, mfma = case
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    units = n * KVH * (-(-(H // KVH) // 16)) * (ctx // 16 + 2)  # MFMA: 16 tokens, 2 start-up units
+    plan = min(cus * (4 if D > 64 else 8), (units // 2 + 3) // 4 * 4)
+    waves = PA.auto_waves(n, H, D, KVH, ctx // 16, 16, W.FP32)
+    print(f"case {case}: {waves} wavefronts, {plan} on the matrix tiles", flush=True)
+    assert (waves == plan) == mfma
+    lens = [max(1, min(ctx, 97) - 7 * i % 90) for i in range(n)]
+    wl = W.small_case(num_seqs=n, H=H, KVH=KVH, D=D, kv_dtype=W.FP32, seed=n + ctx, lens=lens)
+    _check(wl, f"fp32 rule {case}", tokens=ctx)
 
 
 @pytest.mark.parametrize("n", [2, 31, 33, 130, 1025])

@@ -328,22 +328,54 @@ constexpr long long kMaxLaunchTiles = 1LL << 30;  // bounds the partial workspac
 // so each wavefront's range is exactly partition_tokens of K/V.
 constexpr int kSegmentCost = 2;
 
+// Whether an automatic fp32 plan takes the MFMA tiles.  The VALU tile waits
+// for its loads before it computes, works per query head, and reads K/V once
+// per 8 of them; the MFMA tile costs the same for up to 16 heads, with the
+// next tile in flight, but its chain is longer, and rows above 256 bytes run
+// one wavefront per SIMD: ~16 us a step at the least (head_size 128), where
+// the VALU tiles take 11-14 us.  So the real work has to be large enough, and
+// only the table bounds it: the lines lie where a half-filled table does not
+// lose.  Measured on MI355X, both builds in turn on the same tensors, VALU
+// tiles -> MFMA tiles, us a step, for tables filled by a 16th / a quarter /
+// half / all (the longest sequence; the shortest has a quarter of it):
+//   group 4, head_size 128, 32 / 8 heads:
+//     8 seqs, 128 MB    11.5->15.7  14.6->17.1  19.0->19.6  27.7->24.3
+//     8 seqs, 512 MB    14.4->17.1  28.0->24.3  39.1->36.6  64.5->59.5
+//     32 seqs, 512 MB   14.8->17.1  26.6->26.1  38.6->37.9  64.0->60.0
+//     128 seqs of 240, 256 MB  12.0->11.4  20.1->20.8  26.4->28.5  40.5->37.9
+//     128 seqs of 976, 1 GB    20.2->20.9  40.9->38.1  67.1->60.9
+//   (group 3 the same or slightly worse: 32 seqs, 512 MB 13.9->17.0
+//   25.9->25.8  37.6->36.8  63.5->59.7)
+//   group 4, head_size 64, 16 / 4 heads:
+//     32 seqs, 128 MB   12.0->12.9  14.4->15.1  18.0->18.7  25.5->23.4
+//     32 seqs, 256 MB   12.1->13.0  18.0->18.5  25.6->23.2  36.6->35.0
+//   group 8, head_size 128, 64 / 8 heads:
+//     1 seq, 16 MB      13.4->14.6  13.6->15.8  14.2->16.4  15.6->16.7
+//     8 seqs, 32 MB     14.2->11.8  14.2->16.1  15.2->16.7  19.3->17.1
+//     8 seqs, 64 MB     13.7->15.0  15.2->16.7  19.2->17.2  24.7->19.9
+//     32 seqs of 112, 32 MB    11.4->10.1  14.5->12.0  15.3->15.1  19.0->16.3
+//     32 seqs of 48, 16 MB     11.2->9.8   13.0->9.8   14.4->11.7  15.4->15.1
+//     32 seqs, 512 MB   19.2->16.6  34.5->25.7  47.9->37.0  78.6->59.8
+//   group 16, 64 / 4 heads, 32 seqs, 256 MB 19.3->16.6 34.5->20.6 47.5->26.9
+//     78.2->37.5; group 6, head_size 64: 0.73-0.94 of the VALU tiles' time at
+//     every size (4 MB to 1 GB).
+// Groups of 1 and 2 stay on the VALU tiles: full tables of 256 MB and more
+// took 0.95-1.0 of their time (113 -> 107 us), but part-filled ones and many
+// short sequences up to 1.7 times (32 / 32 heads, 32 seqs, 256 MB, a quarter
+// full 15.2 -> 20.3; 128 full sequences of 112 60.5 -> 65.2).
+bool f32_mfma(int heads, int head_size, double table_bytes, long long max_ctx) {
+    const bool long_rows = 4 * head_size > 256;
+    if (heads <= 2) return false;
+    if (heads <= 4)
+        return long_rows ? table_bytes >= 512e6 && max_ctx >= 512 : table_bytes >= 256e6;
+    // (short sequences: few tiles in any wavefront's chain)
+    return !long_rows || table_bytes >= (max_ctx <= 112 ? 16e6 : 64e6);
+}
+
 // Whether an automatic plan of a use_mfma_auto shape takes the MFMA tiles.
 // Not where the batch takes the segment launch (whole outputs only), nor
 // where its 16-token tiles would pass the limit of split units that the VALU
-// tile's longer ones keep.  Else by group and by the K/V bytes the table
-// bounds.  The VALU tile waits for its loads before it computes, works per
-// query head, and reads K/V once per 8 of them; the MFMA tile costs the same
-// for up to 16 heads, with the next tile in flight, but its chain is longer,
-// so short batches of small groups stay.  Measured on MI355X (fp32, VALU ->
-// MFMA tiles, us a step):
-//   group 8, head_size 128: 1 x 96 tokens 13.2 -> 11.7, 8 sequences of
-//     300-900 tokens 25.6 -> 18.8; group 16, 32 of 64-2048: 69.6 -> 34.1;
-//   group 4: bounds of 15-30 MB 13.2 -> 14.2, 14.8 -> 15.8, 15.0 -> 15.7;
-//     59-65 MB 17.8 -> 17.0, 19.8 -> 18.3, 21.6 -> 20.3; 32 sequences of
-//     256-2048 tokens 64.4 -> 57.2;
-//   groups 1 and 2: 63-74 MB 14.4 -> 18.9, 16.8 -> 18.7; 109 MB 27.6 -> 27.1;
-//     218 MB 43.1 -> 38.9.
+// tile's longer ones keep.  fp32: f32_mfma.
 // fp16/bf16, with the weights in fp32 as on the VALU tiles (32 fp32 MFMAs a
 // tile: beside HBM they count from ~40 us on).  Head_size 80 from groups of 3
 // (24 / 8 and 32 / 8 heads, 1-128 sequences, tables of 4 MB to 1 GB filled by
@@ -361,11 +393,10 @@ bool auto_mfma(int kv_dtype, int head_size, int block_size, const HeadTiling &va
     const int heads = valu.head_tile * valu.head_tiles;  // the group, rounded up
     if (kv_dtype != NXT_KV_FP32) {
         if (heads <= (head_size == 80 ? 2 : 4)) return false;
-    } else if (heads <= 4) {
-        constexpr double kMinBytes = 32e6, kMinBytesNarrow = 128e6;
+    } else {
         const double bytes = 2.0 * elem_bytes(kv_dtype) * head_size * num_kv_heads *
                              (double)num_seqs * (double)max_ctx;
-        if (bytes < (heads <= 2 ? kMinBytesNarrow : kMinBytes)) return false;
+        if (!f32_mfma(heads, head_size, bytes, max_ctx)) return false;
     }
     HeadTiling t;
     if (!head_tiling(heads, true, kv_dtype, head_size, &t)) return false;
