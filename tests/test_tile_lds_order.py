@@ -78,3 +78,17 @@ def test_lds_exchange_is_fenced(listing, name):
             if not now <= since.get(b, set()):
                 since[b] = since.get(b, set()) | now
                 work.append(b)
+
+
+def test_cascade_plan_has_its_lds():
+    """The static LDS of the cascade's partition launch leaves the in-kernel
+    plan the room of batches of 1024 to 1500 sequences (larger ones go to the
+    plan kernels, two more launches)."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("no hipcc")
+    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "--offload-device-only", "-fsyntax-only",
+                        "-std=c++17", "-I" + os.path.join(ROOT, "include"),
+                        "-I" + os.path.join(ROOT, "xllms_amd", "csrc"),
+                        os.path.join(ROOT, "tests", "c", "cascade_lds_size.hip")],
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]

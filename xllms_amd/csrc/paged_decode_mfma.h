@@ -905,31 +905,38 @@ __device__ __forceinline__ void fix_absorb(const MfmaFixSlot<KV, D> &slot, int l
 }
 
 // The workgroup's relay slot of the mode-2 combine: one state of R row
-// blocks in the lane layout, and per wavefront whether it relayed its state
-// there (and whether that state reaches the end of its segment).
+// blocks in the lane layout.
 template <int KV, int D, int R> struct MfmaRelaySlot {
     f32x4 o[R][MfmaGeometry<KV, D>::kDimBlocks][64];
     float m[R][64], l[R][64];
-    int relayed[kMfmaWavesPerGroup];
-    int ends[kMfmaWavesPerGroup];
 };
 
-// LDS of one workgroup of the partition kernel: the query rows of
-// each wavefront's piece (R = 2), its V tile (short rows), and the slots of the workgroup-level combine (by
-// mode).
-template <int FIX, int KV, int D, int R> struct MfmaSweepLds {
-    int unused;
-};
-template <int KV, int D, int R> struct MfmaSweepLds<1, KV, D, R> {
-    MfmaFixSlot<KV, D> fix[kMfmaWavesPerGroup];
-};
-template <int KV, int D, int R> struct MfmaSweepLds<2, KV, D, R> {
-    MfmaRelaySlot<KV, D, R> relay;
-};
+// LDS of one workgroup of the partition kernel: the query rows of each
+// wavefront's piece (mfma_q_in_lds), its V tile (short rows), and the slots of
+// the workgroup-level combine (by mode).  Mode 2: the relay slot takes the
+// query rows' place, which no wavefront reads past the combine's first
+// barrier, and beside it, per wavefront, whether it relayed its state and
+// whether that state reaches the end of its segment.  (With a place of its
+// own the slot left the cascade's in-kernel plan 30 KB for two workgroups per
+// CU, not 46: 64 / 1 heads, 720 sequences in 16 groups went to the plan
+// kernels, 143 us a step for 131.)
 template <int KV, int D, int R, int FIX = mfma_wg_fixup(kMfmaHeads * R, D)> struct MfmaLds {
     MfmaQLds<KV, D, R> qs[kMfmaWavesPerGroup];
     MfmaVLds<KV, D> vs[kMfmaWavesPerGroup];
-    MfmaSweepLds<FIX, KV, D, R> sw;
+};
+template <int KV, int D, int R> struct MfmaLds<KV, D, R, 1> {
+    MfmaQLds<KV, D, R> qs[kMfmaWavesPerGroup];
+    MfmaVLds<KV, D> vs[kMfmaWavesPerGroup];
+    MfmaFixSlot<KV, D> fix[kMfmaWavesPerGroup];
+};
+template <int KV, int D, int R> struct MfmaLds<KV, D, R, 2> {
+    union {
+        MfmaQLds<KV, D, R> qs[kMfmaWavesPerGroup];
+        MfmaRelaySlot<KV, D, R> relay;
+    };
+    MfmaVLds<KV, D> vs[kMfmaWavesPerGroup];
+    int relayed[kMfmaWavesPerGroup];
+    int ends[kMfmaWavesPerGroup];
 };
 
 // st <- st (+) the partial in workspace slot `slot` (its l is the reduced
@@ -1042,7 +1049,7 @@ __device__ __forceinline__ void mfma_partition_body(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if constexpr (FIX == 2) {
         // ordered before any read by the sweep's first barrier
-        if (lane == 0) sm.sw.relay.relayed[wave] = 0;
+        if (lane == 0) sm.relayed[wave] = 0;
     }
 
     const int B = p.num_seqs;
@@ -1173,8 +1180,8 @@ __device__ __forceinline__ void mfma_partition_body(
                     // (whose left neighbour is in another workgroup) is
                     // written as a partial after the range, so that its
                     // stores do not sit in front of the next piece's loads.
-                    fix_store<KV, D>(sm.sw.fix[wave], lane, st[0]);
-                    if (lane == 0) sm.sw.fix[wave].ends = 1;
+                    fix_store<KV, D>(sm.fix[wave], lane, st[0]);
+                    if (lane == 0) sm.fix[wave].ends = 1;
                     if (wave == 0) {
                         pc_first = pc;
                         first_saved = true;
@@ -1204,27 +1211,28 @@ __device__ __forceinline__ void mfma_partition_body(
 #endif
 
     if constexpr (FIX == 2) {
-        // As below, with the one relay slot.
+        // As below, with the one relay slot (which overlays the query rows:
+        // every wavefront is past its tiles from here on).
         __syncthreads();
         for (int i = NW - 1; i >= 0; i--) {
             if (wave == i && have_last) {
                 const bool cut_start = pc.t_begin > 0;
                 bool ends = pc.t_end >= pc.L;
                 if (!ends && i < NW - 1) {
-                    if (sm.sw.relay.relayed[i + 1]) {
+                    if (sm.relayed[i + 1]) {
 #pragma unroll
                         for (int b = 0; b < R; b++) {
-                            const float mo = sm.sw.relay.m[b][lane];
+                            const float mo = sm.relay.m[b][lane];
                             const float M = fmaxf(st[b].m, mo);
                             const float Ms = (M == -INFINITY) ? 0.0f : M;
                             const float a = fast_exp2(st[b].m - Ms), wt = fast_exp2(mo - Ms);
-                            st[b].l = st[b].l * a + sm.sw.relay.l[b][lane] * wt;
+                            st[b].l = st[b].l * a + sm.relay.l[b][lane] * wt;
 #pragma unroll
                             for (int n = 0; n < G::kDimBlocks; n++)
-                                st[b].o[n] = st[b].o[n] * a + sm.sw.relay.o[b][n][lane] * wt;
+                                st[b].o[n] = st[b].o[n] * a + sm.relay.o[b][n][lane] * wt;
                             st[b].m = M;
                         }
-                        ends = sm.sw.relay.ends[i + 1] != 0;
+                        ends = sm.ends[i + 1] != 0;
                     } else {
                         // the neighbour's first piece, followed by more
                         // pieces, was written as a partial in its slot 0;
@@ -1237,13 +1245,13 @@ __device__ __forceinline__ void mfma_partition_body(
 #pragma unroll
                     for (int b = 0; b < R; b++) {
 #pragma unroll
-                        for (int n = 0; n < G::kDimBlocks; n++) sm.sw.relay.o[b][n][lane] = st[b].o[n];
-                        sm.sw.relay.m[b][lane] = st[b].m;
-                        sm.sw.relay.l[b][lane] = st[b].l;
+                        for (int n = 0; n < G::kDimBlocks; n++) sm.relay.o[b][n][lane] = st[b].o[n];
+                        sm.relay.m[b][lane] = st[b].m;
+                        sm.relay.l[b][lane] = st[b].l;
                     }
                     if (lane == 0) {
-                        sm.sw.relay.relayed[i] = 1;
-                        sm.sw.relay.ends[i] = ends ? 1 : 0;
+                        sm.relayed[i] = 1;
+                        sm.ends[i] = ends ? 1 : 0;
                     }
                 } else if (!cut_start && ends) {
                     mfma_write_rows<KV, D, R, HS>(p, pc, lane, st);
@@ -1265,20 +1273,20 @@ __device__ __forceinline__ void mfma_partition_body(
         // finished rows when it lay in the workgroup, else one partial.
         const bool cut_start = have_last && pc.t_begin > 0;
         if (have_last && cut_start && wave > 0) {
-            fix_store<KV, D>(sm.sw.fix[wave], lane, st[0]);
-            if (lane == 0) sm.sw.fix[wave].ends = pc.t_end >= pc.L ? 1 : 0;
+            fix_store<KV, D>(sm.fix[wave], lane, st[0]);
+            if (lane == 0) sm.fix[wave].ends = pc.t_end >= pc.L ? 1 : 0;
         }
         __syncthreads();
         if (first_saved) {
             MfmaState<KV, D> sf[R];
-            fix_load<KV, D>(sm.sw.fix[0], lane, sf[0]);
+            fix_load<KV, D>(sm.fix[0], lane, sf[0]);
             mfma_write_partial<KV, D, R, HS>(p, pc_first, lane, sf);
         }
         if (have_last && !(cut_start && wave > 0)) {
             bool ends = pc.t_end >= pc.L;
             for (int j = wave + 1; !ends && j < NW; j++) {
-                fix_absorb<KV, D>(sm.sw.fix[j], lane, st[0]);
-                ends = sm.sw.fix[j].ends != 0;
+                fix_absorb<KV, D>(sm.fix[j], lane, st[0]);
+                ends = sm.fix[j].ends != 0;
             }
             if (!cut_start && ends)
                 mfma_write_rows<KV, D, R, HS>(p, pc, lane, st);
