@@ -22,6 +22,7 @@ template <int KV, int D> constexpr bool fits() {
            plan_bytes(1024, 16, 256) <= plan_room<KV, D, 1>();
 }
 static_assert(fits<KV_F16, 128>() && fits<KV_BF16, 128>(), "head_size 128");
+static_assert(fits<KV_F16, 96>() && fits<KV_BF16, 96>(), "head_size 96");
 static_assert(fits<KV_F16, 64>() && fits<KV_F16, 32>(), "head_sizes 64 and 32");
 
 }  // namespace xhip

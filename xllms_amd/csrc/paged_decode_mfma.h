@@ -247,9 +247,11 @@ template <int KV, int D> struct MfmaState {
 // A piece's query rows (MFMA B layout): in registers, or, where R = 2 states
 // leave no room for them beside two tiles of K/V (head_size 128: 10 VGPRs
 // spilled, and 64 / 2 heads over 64 sequences of 512-8192 tokens took 76.7 us
-// against 67.0), parked by each lane in LDS and read back every tile.
+// against 67.0), parked by each lane in LDS and read back every tile.  At
+// head_size 96 they fit, and LDS is the slower place (64 / 2 heads, 32
+// sequences of 650-2592 tokens 25.5 us against 22.3).
 template <int KV, int D, int R> constexpr bool mfma_q_in_lds() {
-    return R == 2 && MfmaGeometry<KV, D>::kRowBytes > 128;
+    return R == 2 && MfmaGeometry<KV, D>::kRowBytes > 192;
 }
 template <int KV, int D, int R, bool LDS = mfma_q_in_lds<KV, D, R>()> struct MfmaQLds {};
 template <int KV, int D, int R> struct MfmaQLds<KV, D, R, true> {
