@@ -14,9 +14,9 @@
 // own stream-K plan.  Every workgroup scans the split units of
 // both batches (LDS) and takes the same split: the prefix batch gets a share
 // of the workgroups proportional to its wavefront-units (a prefix unit
-// occupies a pair of wavefronts) weighted by kCascadeUnitCost, plus the
+// occupies a pair of wavefronts) weighted by cascade_unit_cost, plus the
 // workgroups the suffix plan would leave empty.  Measured on MI355X at
-// config 5 (cascade step, in-kernel plan, one box): weights 0.65 / 0.75 /
+// config 5 (head_size 128; cascade step, in-kernel plan, one box): weights 0.65 / 0.75 /
 // 0.85 gave 121.3-121.5 / 111.6-111.7 / 114.4-114.5 us (86 / 97 / 108 prefix
 // workgroups of 512); without the empty suffix workgroups moved over, 0.85
 // (99) gave 113.2-113.3 us.  The step is sensitive to the split: both
@@ -52,11 +52,22 @@
 namespace xhip {
 
 // Weight of a prefix-batch split unit against a suffix-batch unit in the
-// workgroup split, in percent.
-#ifndef XHIP_CASCADE_UNIT_COST
-#define XHIP_CASCADE_UNIT_COST 75
-#endif
-constexpr int kCascadeUnitCost = XHIP_CASCADE_UNIT_COST;
+// workgroup split, in percent, by the element type, the bytes of a K row and
+// the suffix batch's row blocks (rs).  A prefix unit is a tile for two row
+// blocks; a suffix unit with two costs nearly as much, and what makes a
+// prefix unit cheaper is that its shared pages come from the cache.  Rows of
+// 256 bytes wait longest for HBM; shorter ones pass V through LDS, and their
+// tiles' own work counts for more; over bf16 the prefix states are fp32.
+// Measured on MI355X, 6 batches of 64-320 sequences in 4-30 groups for each
+// of 1 to 64 query heads per kv head, geometric mean of the step against a
+// weight of 75 throughout: rs = 1, head_size 32 fp16 / bf16 0.95 / 0.94, 64
+// 0.96 / 1.0, 96 0.97 / 0.95, 128 bf16 0.99; rs = 2, head_size 128 0.95 /
+// 0.92, below 128 0.98.  (With 75, 64 / 1 heads at head_size 128 in bf16 took
+// up to 1.2 times what it did before the tiles changed.)
+constexpr int cascade_unit_cost(int kv, int row_bytes, int rs) {
+    if (rs == 2) return row_bytes < 256 ? 62 : 50;
+    return row_bytes < 256 ? 95 : kv == KV_F16 ? 75 : 88;
+}
 
 // Workgroups of the prefix body in a launch of G >= 2 workgroups, from the
 // split units of the prefix (tp) and suffix (ts) batches: each batch with
@@ -65,11 +76,12 @@ constexpr int kCascadeUnitCost = XHIP_CASCADE_UNIT_COST;
 // last workgroups nothing: those go to the prefix body, whose ranges get
 // shorter while the suffix's stay the same.  Integer arithmetic only: every
 // workgroup computes the same split.
-__device__ __forceinline__ int cascade_prefix_groups(int tp, int ts, int G, int min_tpw) {
+__device__ __forceinline__ int cascade_prefix_groups(int tp, int ts, int G, int min_tpw,
+                                                     int cost) {
     if (tp <= 0) return 0;
     if (ts <= 0) return G;
     // a prefix unit occupies both wavefronts of a pair
-    const long long a = 2LL * tp * kCascadeUnitCost, b = (long long)ts * 100;
+    const long long a = 2LL * tp * cost, b = (long long)ts * 100;
     int gp = (int)((a * G + (a + b) / 2) / (a + b));
     gp = gp < 1 ? 1 : (gp > G - 1 ? G - 1 : gp);
     const int ws = (G - gp) * kMfmaWavesPerGroup;
@@ -119,7 +131,8 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, 2) void paged_decode_casca
     batch_prefix<16, NW>(ps, pre_s);
     const int G = gridDim.x;
     const int gp = cascade_prefix_groups(pre_p[pp.num_seqs], pre_s[ps.num_seqs], G,
-                                         ps.min_tiles_per_wave);
+                                         ps.min_tiles_per_wave,
+                                         cascade_unit_cost(KV, MfmaGeometry<KV, D>::kRowBytes, RS));
     // neighbouring logical workgroups share an XCD (and its L2).  (Giving
     // every XCD its share of prefix workgroups instead measured 0.5-1 us
     // slower.)
@@ -290,7 +303,8 @@ __global__ __launch_bounds__(64 * kMfmaWavesPerGroup, 2) void paged_decode_casca
     XHIP_WG_STAMP(pp, 18);
     // 4.
     const int Gw = gridDim.x;
-    const int gp = cascade_prefix_groups(pre_p[V], pre_s[B], Gw, ps.min_tiles_per_wave);
+    const int gp = cascade_prefix_groups(pre_p[V], pre_s[B], Gw, ps.min_tiles_per_wave,
+                                         cascade_unit_cost(KV, MfmaGeometry<KV, D>::kRowBytes, RS));
     const int l = xcd_local_block(blockIdx.x, Gw);
     if (blockIdx.x == 0) {
         for (int v = tid; v <= V; v += NT) pp.ws_prefix[v] = pre_p[v];
