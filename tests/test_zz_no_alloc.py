@@ -11,6 +11,7 @@ output.
 from __future__ import annotations
 
 import ctypes
+import dataclasses
 
 import numpy as np
 import pytest
@@ -99,6 +100,26 @@ def test_largest_automatic_plans_fit(cuda, shape):
     a, b = _both(small)
     assert np.array_equal(a, b)
     assert_close(a, O.run_workload(small, precision="mt"), W.FP32, "noalloc fp32 small")
+
+
+def test_explicit_plan_that_just_fits(cuda):
+    """An explicit plan whose partials and unit prefix (one entry per
+    sequence, and the total) fill 66 MiB to the byte: 127 sequences of 11
+    heads, head_size 32 in fp32, tables of 1457 pages of 32 tokens, 256-token
+    ranges: 254432 wavefronts, 2 x 272 bytes of partials each.  What the
+    kernels keep beside them does not count against the plan."""
+    import torch
+    lens = [1 + (37 * i) % 600 for i in range(127)]
+    wl = W.small_case(num_seqs=127, H=11, KVH=11, D=32, bs=32, kv_dtype=W.FP32, seed=15, lens=lens)
+    tables = np.full((127, 1457), -1, dtype=np.int32)
+    tables[:, : wl.block_tables.shape[1]] = wl.block_tables
+    wl = dataclasses.replace(wl, block_tables=tables)
+    assert wl.max_num_blocks_per_seq == 1457
+    print("case noalloc, a plan of 66 MiB", flush=True)
+    a, b = _both(wl, part=256)
+    assert np.array_equal(a, b)
+    assert_close(a, O.run_workload(wl, precision="mt"), W.FP32, "noalloc, 66 MiB")
+    torch.cuda.synchronize()
 
 
 def test_no_device_allocation(cuda):

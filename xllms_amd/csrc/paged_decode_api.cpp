@@ -611,9 +611,11 @@ int run(void *out, const void *query, const void *key_cache, const void *value_c
         }
 
         const size_t eb_total = (size_t)elem_bytes(kv_dtype);
-        // workspace: fp32 partials o, their (m, l), the unit prefix; under a
-        // split segment launch, one partial per workgroup
-        const size_t pre_bytes = seg_launch ? 0 : (size_t)(nseq + 2) * sizeof(int);
+        // workspace: fp32 partials o, their (m, l), the unit prefix and, after
+        // it, the units per wavefront (one int, in the fixed scratch's tail);
+        // under a split segment launch, one partial per workgroup
+        const size_t pre_bytes = seg_launch ? 0 : (size_t)(nseq + 1) * sizeof(int);
+        const size_t tail_bytes = seg_launch ? 0 : sizeof(int);
         long long slots = seg_launch ? (seg_split > 1 ? nseq * segs * seg_split : 0)
                                      : 2 * waves;
         auto o_size = [&](long long n) {
@@ -654,7 +656,7 @@ int run(void *out, const void *query, const void *key_cache, const void *value_c
         } else if (fixed) {
             ws = fixed->ptr;  // launches of one stream run in order: chunks reuse it
         } else {
-            int st = get_workspace(device, stream, o_bytes + ml_bytes + pre_bytes, &lease);
+            int st = get_workspace(device, stream, o_bytes + ml_bytes + pre_bytes + tail_bytes, &lease);
             if (st != NXT_ATTN_OK) return st;
             ws = lease.ptr();
         }

@@ -17,7 +17,7 @@
 
 namespace {
 
-static __device__ __align__(256) char scratch[xhip::kNoAllocScratchBytes];
+static __device__ __align__(256) char scratch[xhip::kNoAllocScratchBytes + xhip::kNoAllocScratchTail];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
