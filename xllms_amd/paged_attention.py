@@ -68,10 +68,13 @@ def _ptr(t) -> int:
 def _stream_handle(stream) -> int:
     if stream is None:
         # the current stream's handle without building a Stream object around
-        # it (the operators' host time is what bounds their smallest calls)
+        # it (the operators' host time is what bounds their smallest calls),
+        # where this torch has the two calls for it, which are not public
         import torch
-        if torch.cuda.is_initialized():
-            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        device = getattr(torch._C, "_cuda_getDevice", None)
+        if raw is not None and device is not None and torch.cuda.is_initialized():
+            return raw(device())
         stream = torch.cuda.current_stream()
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
