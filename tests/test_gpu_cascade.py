@@ -90,13 +90,19 @@ def test_cascade_config5_matches_oracle(cuda):
                                           ("fp32", 128, 32, 8), ("fp16", 96, 64, 2),
                                           ("bf16", 32, 48, 1), ("fp16", 128, 64, 1),
                                           ("bf16", 64, 48, 2), ("bf16", 128, 64, 4),
-                                          ("fp16", 32, 16, 4)])
+                                          ("fp16", 32, 16, 4), ("fp32", 64, 16, 2),
+                                          ("fp32", 96, 32, 2), ("fp32", 32, 20, 1),
+                                          ("fp16", 112, 16, 4), ("fp16", 112, 16, 2),
+                                          ("bf16", 112, 10, 1), ("bf16", 80, 32, 2)])
 def test_cascade_groups_match_oracle(cuda, dtype, D, H, KVH):
     """Groups of 1..21 members (prefix rows spanning several 16- or 32-row
     prefix sequences), members with an empty suffix, unshared sequences
     (L = 1, L = 0, long), on the MFMA (one and two 16-head row blocks per
     wavefront) and VALU tile paths.  On the MFMA path with head_size <= 128
-    the two batches run in one launch with paired prefix head tiles: group 64
+    the two batches run in one launch with paired prefix head tiles (16-bit
+    types, head sizes that are multiples of 32; fp32 and head sizes 80 and 112
+    in two passes, the second folding in the first's fp32 rows, on the VALU or
+    the matrix tiles by the head size and the group): group 64
     fills a 64-row prefix sequence with one member, group 24 splits some
     members' rows between two prefix sequences."""
     spec = [(5, [3, 0, 40, 16, 1]), (1, [7] * 21), (12, [100]), (2, [0, 0])]
@@ -105,6 +111,23 @@ def test_cascade_groups_match_oracle(cuda, dtype, D, H, KVH):
     print(f"case {dtype} D={D} H={H} KVH={KVH}", flush=True)
     assert_close(run_cascade(wl, pg, pb), O.run_workload(wl, precision="mt"), wl.kv_dtype,
                  f"cascade {dtype} D={D}")
+
+
+@pytest.mark.parametrize("D,H,KVH", [(128, 16, 2), (96, 32, 2), (128, 40, 2)])
+def test_cascade_fp32_matrix_tiles(cuda, D, H, KVH):
+    """fp32 at head sizes above 64 under tables wide enough for the matrix
+    tiles (64 MB of K/V bounded): both passes run them, and the second folds
+    in the first's rows after its tiles."""
+    import dataclasses
+    spec = [(5, [3, 0, 40, 16, 1]), (1, [7] * 21), (12, [100]), (2, [0, 0])]
+    wl, pg, pb = shared_case(spec, singles=[1, 0, 333], H=H, KVH=KVH, D=D, kv_dtype=W.FP32,
+                             seed=D + H)
+    tables = np.full((wl.num_seqs, 256), -1, dtype=np.int32)
+    tables[:, : wl.block_tables.shape[1]] = wl.block_tables
+    wl = dataclasses.replace(wl, block_tables=tables)
+    print(f"case fp32 D={D} H={H} KVH={KVH}", flush=True)
+    assert_close(run_cascade(wl, pg, pb), O.run_workload(wl, precision="mt"), W.FP32,
+                 f"cascade fp32 D={D}")
 
 
 def test_cascade_ignores_entries_that_do_not_fit(cuda):

@@ -116,12 +116,16 @@ def test_split_k_every_tile_path(cuda, dtype, head_size):
     (80, 2, 128, "fp16", 128),
     (48, 2, 256, "fp16", 128),
     (12, 1, 128, "fp32", 256),
-    # VALU groups of 17-24 heads: three head tiles of 8, the last partly
-    # filled (fp32 at 128 and 64 dims; bf16 at head_size 80, which the MFMA
-    # path does not take)
+    # groups of 17-24 heads outside the 16-bit multiples of 32: automatic plans
+    # take two matrix head tiles of 16, explicit partitions three VALU tiles
+    # of 8, the last one partly filled either way
     (48, 2, 128, "fp32", 64),
     (40, 2, 64, "fp32", 128),
     (17, 1, 80, "bf16", 256),
+    # and three VALU tiles of 8 in both (fp32 above head_size 128)
+    (48, 2, 192, "fp32", 64),
+    (40, 2, 256, "fp32", 128),
+    (17, 1, 192, "fp32", 256),
 ])
 def test_merge_per_segment_paths(cuda, shape):
     """Batches with enough segments merge with one workgroup per segment:
