@@ -176,7 +176,8 @@ int ilog2(int x) {
 int elem_bytes(int kv_dtype) { return kv_dtype == NXT_KV_FP32 ? 4 : 2; }
 
 // The MFMA tile path serves fp16/bf16 with head_size % 32 == 0 and pages of
-// at least one 16-token tile; every other shape takes the VALU tile path.
+// at least one 16-token tile; of the other shapes, which take the VALU tile
+// path, automatic plans may choose it too (use_mfma_auto).
 bool use_mfma(int kv_dtype, int head_size, int block_size) {
     return kv_dtype != NXT_KV_FP32 && head_size % 32 == 0 && block_size >= 16;
 }

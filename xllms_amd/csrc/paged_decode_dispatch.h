@@ -1,6 +1,7 @@
 // Shared body of the per-dtype launch units: (tile path, head_size, head_tile)
-// dispatch.  The MFMA path exists for the 16-bit types and head sizes that are
-// multiples of 32; the VALU path covers every supported shape.
+// dispatch.  The MFMA path exists for the 16-bit types at every head size and
+// for fp32 at multiples of 32 up to kMfmaF32MaxHeadSize; the VALU path covers
+// every supported shape.
 #pragma once
 
 #include <hip/hip_ext.h>
@@ -64,41 +65,34 @@ static hipError_t launch_partition(F kernel, unsigned grid, unsigned block, size
     return hipGetLastError();
 }
 
+// The per-segment merge of segments of `cols` float4 columns, one thread per
+// column of up to HI = 8, 16, ... 1024 of them: at least a wavefront, whose
+// lanes share the columns below 64.  Instantiated only for the counts that a
+// first head tile can have (a tile of GT holds more than GT / 2 heads, but
+// one of a single row block any number).
+template <int KV, int D, int GT, int TT, int HI = 8>
+static hipError_t launch_merge_segments(const DecodeParams &p, dim3 grid, int cols,
+                                        hipStream_t st) {
+    constexpr int kMinCols = (GT == kMfmaHeads ? 1 : GT / 2 + 1) * (D / 4), kMaxCols = GT * (D / 4);
+    if constexpr (kMinCols <= HI && kMaxCols > HI / 2) {
+        if (cols <= HI) {
+            constexpr int NT = HI < 64 ? 64 : HI;
+            paged_decode_merge_segment_kernel<KV, D, GT, TT, NT, NT / HI>
+                <<<grid, NT, 0, st>>>(p);
+            return hipGetLastError();
+        }
+    }
+    if constexpr (kMaxCols > HI) return launch_merge_segments<KV, D, GT, TT, 2 * HI>(p, grid, cols, st);
+    return hipErrorInvalidValue;
+}
+
 template <int KV, int D, int GT, int TT>
 static hipError_t launch_merge(const DecodeParams &p, hipStream_t st) {
     const unsigned segs = (unsigned)(p.num_kv_heads * p.head_tiles);
     const int heads = p.group < GT ? p.group : GT;
     const int cols = heads * (D / 4);
-    if (p.merge_per_segment) {
-        // one thread per float4 column of the segment (heads * D/4), the
-        // count rounded up to a power of two from 64 to 1024; up to 32
-        // columns, the lanes of one wavefront share them.  Instantiations
-        // exist only where a segment can have that many columns.
-        const dim3 grid(segs, (unsigned)p.num_seqs);
-        constexpr int kMaxCols = GT * (D / 4);
-        constexpr int kNt128 = kMaxCols > 64 ? 128 : 64;
-        constexpr int kNt256 = kMaxCols > 128 ? 256 : 64;
-        constexpr int kNt512 = kMaxCols > 256 ? 512 : 64;
-        constexpr int kNt1024 = kMaxCols > 512 ? 1024 : 64;
-        if (cols <= 8)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, 64, 8><<<grid, 64, 0, st>>>(p);
-        else if (cols <= 16)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, 64, 4><<<grid, 64, 0, st>>>(p);
-        else if (cols <= 32)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, 64, 2><<<grid, 64, 0, st>>>(p);
-        else if (cols <= 64)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, 64, 1><<<grid, 64, 0, st>>>(p);
-        else if (cols <= 128)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt128, 1><<<grid, kNt128, 0, st>>>(p);
-        else if (cols <= 256)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt256, 1><<<grid, kNt256, 0, st>>>(p);
-        else if (cols <= 512)
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt512, 1><<<grid, kNt512, 0, st>>>(p);
-        else
-            paged_decode_merge_segment_kernel<KV, D, GT, TT, kNt1024, 1>
-                <<<grid, kNt1024, 0, st>>>(p);
-        return hipGetLastError();
-    }
+    if (p.merge_per_segment)
+        return launch_merge_segments<KV, D, GT, TT>(p, dim3(segs, (unsigned)p.num_seqs), cols, st);
     const dim3 grid(segs, (unsigned)((cols + kMergeCols - 1) / kMergeCols), (unsigned)p.num_seqs);
     // the new-token fold needs a head's columns in one aligned lane group
     constexpr bool kFold = D == 32 || D == 64 || D == 128;

@@ -946,14 +946,6 @@ __device__ __forceinline__ f32x4 unpack_h4(u32x2 h) {
     return f32x4{a.x, a.y, b.x, b.y};
 }
 
-// Four consecutive values of a partial's o at float index `at` of the
-// split-K workspace: fp32, or HS: fp16 states (DecodeParams::ws_h).
-template <bool HS>
-__device__ __forceinline__ f32x4 partial_f32x4(const DecodeParams &p, size_t at) {
-    if constexpr (HS) return unpack_h4(*(const u32x2 *)((const char *)p.ws_h + at * 2));
-    else return *(const f32x4 *)(p.ws_o + at);
-}
-
 // Online log-sum-exp merge, into (m, l, acc) of one float4 column, of a
 // segment's partials j = j0, j0 + step, ... < np (slots as in PartialSlots).
 // The partials go in batches of up to NB whose loads are all issued before
