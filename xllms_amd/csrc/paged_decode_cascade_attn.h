@@ -103,7 +103,8 @@ template <int KV, int D, int RS> union MfmaLdsPair {
 // The units per range of both batches, for the merge (in place of its own
 // divisions: its code comes from a cold cache, and at 3.9 KB instead of 6.2 a
 // step over 256 sequences in 16 groups, fp16, takes 108.3 us instead of
-// 109.5), stored after the workgroup's ranges.  tp / ts: the batches' units; gp of G workgroups are the prefix's.
+// 109.5), stored after the workgroup's ranges.  tp / ts: the batches' units;
+// gp of G workgroups are the prefix's.
 __device__ __forceinline__ void cascade_publish_ranges(const DecodeParams &pp,
                                                        const DecodeParams &ps, int tp, int ts,
                                                        int gp, int G) {

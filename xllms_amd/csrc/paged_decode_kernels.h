@@ -950,7 +950,7 @@ __device__ __forceinline__ f32x4 unpack_h4(u32x2 h) {
 // segment's partials j = j0, j0 + step, ... < np (slots as in PartialSlots).
 // The partials go in batches of up to NB whose loads are all issued before
 // any is used, so a thread waits for one memory round trip per batch, not
-// per partial; batch slots past np load and combine nothing.  A batch is
+// per partial; batch slots past np load nothing and weigh 0.  A batch is
 // combined under its largest running max: one exponential and five
 // multiply-adds per partial.  The column's (m, l) and float4 of o sit at
 // off_ml and off_o floats into a slot.  HS: fp16 states (DecodeParams::ws_h),

@@ -49,9 +49,10 @@ constexpr int kSegTiles = 2;
 constexpr int kSegRounds = 4;
 constexpr int kSegMaxHeadTile = 2;
 
-// Workgroup-level combine of cut segments (MFMA tile path): the kMfmaWavesPerGroup wavefronts of a workgroup own consecutive
-// stream-K ranges, so the pieces of one segment that fall in one workgroup
-// are merged through LDS at the end of the kernel.  Only one fp32 partial
+// Workgroup-level combine of cut segments (MFMA tile path): the
+// kMfmaWavesPerGroup wavefronts of a workgroup own consecutive stream-K
+// ranges, so the pieces of one segment that fall in one workgroup are merged
+// through LDS at the end of the kernel.  Only one fp32 partial
 // per (segment, workgroup it spans) is left for the merge kernel, in the
 // slot of the leftmost wavefront holding a piece of it, and a segment lying
 // inside one workgroup is written finished.  Mode 1 (one row block): every
@@ -69,12 +70,10 @@ constexpr int mfma_wg_fixup(int rows_per_tile, int head_size) {
 // launches in one resident round, by the bytes of a K (or V) row: about 64 KB
 // of tiles per CU, twice that with the next tiles in flight.  Rows of 128 to
 // 256 bytes: two; three measured 4-10% slower at 256 bytes (more page streams
-// per HBM channel), 2% at 128.  Longer rows (16 KB tiles): one; two had HBM
-// serve them unevenly (fp32, head_size 128, 32 / 8 heads, 32 sequences of
-// 256-2048 tokens: the wavefronts' last tiles spread over 41-60 us, 67.5 us a
-// step; one per SIMD 46-52 us, 57.8 us).  64-byte rows (2 KB tiles), one row
-// block: four (bf16, head_size 32, 32 / 8 heads, 64 sequences of 256-4096
-// tokens: 38.1 -> 32.6 us).
+// per HBM channel), 2% at 128.  Longer rows (16 KB tiles): one (fp32,
+// head_size 128, 32 / 8 heads, 32 sequences of 256-2048 tokens 57.8 us a step;
+// two 67.5).  64-byte rows (2 KB tiles), one row block: four (bf16, head_size
+// 32, 32 / 8 heads, 64 sequences of 256-4096 tokens: 38.1 -> 32.6 us).
 constexpr int mfma_waves_per_simd(int row_bytes, int rows_per_tile) {
     return row_bytes > 256 ? 1 : row_bytes <= 64 && rows_per_tile == kMfmaHeads ? 4 : 2;
 }
