@@ -82,6 +82,16 @@ template <int KV, int D> struct MfmaGeometry {
     // too: two 16-bit parts are ~22 bits of P for fp16, 16 for bf16, and a V
     // of infinity times a part that is 0 is NaN.
     static constexpr bool kP32 = KV == KV_F32 || kPadded;
+    // Its MFMAs of four tokens per chain of a tile's sum.  fp32 results hold
+    // the rounding of that sum, and chains of 16 tokens left short contexts
+    // further from 64 bits than the VALU tiles, which add up 4 to 8 rows' sums
+    // (16 tokens: head_size 64 1.18e-7 against 1.13e-7, 128 1.23e-7 against
+    // 1.19e-7).  Two chains of 8: 1.09e-7 and 1.15e-7, and 1.86e-7 against
+    // 2.05e-7 at 2000 tokens, for 0.7% of the step of 32 sequences of up to
+    // 2048 tokens at 32 / 8 heads, 1-3% at more heads.  Four of 4 (3% more)
+    // where the VALU tiles add up the most rows, head_size 32: 1.09e-7 against
+    // 1.11e-7; chains of 16 had 1.19e-7.  16-bit results show none of this.
+    static constexpr int kPvChain = KV != KV_F32 ? 4 : kRowBytes < 256 ? 1 : 2;
     static constexpr int group_words(int b) { return group_dims(b) * kElemBytes / 4; }
     static constexpr int kDimBlocks = kDims * (kVGroups - 1) + group_dims(kVGroups - 1);
     // Rows of fewer than 16 chunks of 16 bytes: the tile is loaded in whole
@@ -445,11 +455,14 @@ __device__ __forceinline__ void mfma_tile(const DecodeParams &p, const MfmaQuery
         for (int e = 0; e < G::group_dims(B); e++) {
             if constexpr (G::kP32) {
                 f32x4 &o = st[0].o[G::kDims * B + e];
-                f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+                f32x4 t[4];
 #pragma unroll
                 for (int i = 0; i < 4; i++)
-                    t = mfma_f32(chunk_elem<KV>(v[i], e), __builtin_bit_cast(uint32_t, p32[i]), t);
-                o = o * alpha32 + t;
+                    t[i] = mfma_f32(chunk_elem<KV>(v[i], e), __builtin_bit_cast(uint32_t, p32[i]),
+                                    i % G::kPvChain == 0 ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : t[i - 1]);
+                if constexpr (G::kPvChain == 4) o = o * alpha32 + t[3];
+                else if constexpr (G::kPvChain == 2) o = o * alpha32 + (t[1] + t[3]);
+                else o = o * alpha32 + ((t[0] + t[1]) + (t[2] + t[3]));
                 continue;
             }
             const int n = G::kDims * B + e, w = e / 2;
